@@ -226,23 +226,30 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // select of the source addresses, so the loop has no branch. Every lane loads (activation
   // rows and scale rows past the item's end repeat its first row into slots nobody reads), so
   // no load is divergent; every wave loads even if it has no rows.
-  auto issue = [&](int kk, int s) __attribute__((always_inline)) {
+  // Loads [from, to) of the step's S::kLoadsPerStep.
+  auto issue_some = [&](int kk, int s, int from, int to) __attribute__((always_inline)) {
     const bool nxt = !G1 && kk >= KS && have_n;
     const int k = kk < KS ? kk : (nxt ? kk - KS : KS - 1);
     TileStage<ROWS>& st = sh.st[s];
     const uint8_t* wk = (nxt ? n.wbase : c.wbase) + k * 128;
 #pragma unroll
-    for (int j = 0; j < kWDma; ++j) dma16(wk + (nxt ? n.woff[j] : c.woff[j]), &st.w[(32 * wave + 8 * j) * 128]);
+    for (int j = 0; j < kWDma; ++j)
+      if (from <= j && j < to) dma16(wk + (nxt ? n.woff[j] : c.woff[j]), &st.w[(32 * wave + 8 * j) * 128]);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) dma16((nxt ? n.asrc[j] : c.asrc[j]) + k * 128, &st.a[8 * (wave + kTileWaves * j) * 128]);
-    const float* sk = (nxt ? n.ssrc : c.ssrc) + k * c.sstride;
-    if constexpr (S::kThirdBlock) {
-      if (wave < 4) dma16((nxt ? n.asrc[2] : c.asrc[2]) + k * 128, &st.a[8 * (wave + 2 * kTileWaves) * 128]);
-      else dma4(sk, &st.sa[64 * c.sblk]);
-    } else {
-      dma4(sk, &st.sa[S::kSSlots * c.shalf + 64 * c.sblk]);
+    for (int j = 0; j < 2; ++j)
+      if (from <= kWDma + j && kWDma + j < to)
+        dma16((nxt ? n.asrc[j] : c.asrc[j]) + k * 128, &st.a[8 * (wave + kTileWaves * j) * 128]);
+    if (from <= kWDma + 2 && kWDma + 2 < to) {
+      const float* sk = (nxt ? n.ssrc : c.ssrc) + k * c.sstride;
+      if constexpr (S::kThirdBlock) {
+        if (wave < 4) dma16((nxt ? n.asrc[2] : c.asrc[2]) + k * 128, &st.a[8 * (wave + 2 * kTileWaves) * 128]);
+        else dma4(sk, &st.sa[64 * c.sblk]);
+      } else {
+        dma4(sk, &st.sa[S::kSSlots * c.shalf + 64 * c.sblk]);
+      }
     }
   };
+  auto issue = [&](int kk, int s) __attribute__((always_inline)) { issue_some(kk, s, 0, S::kLoadsPerStep); };
 
   constexpr int NG1 = NG > 0 ? NG : 1;
   v4f acc[W32 ? 1 : 4][W32 ? 1 : NG1];
@@ -314,7 +321,16 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   v4f dp[4] = {zero, zero, zero, zero};
   float p0 = 0.f, p1 = 0.f;
 
-  auto compute = [&](int s, const Head& h, float s0, float s1) __attribute__((always_inline)) {
+  // A step's loads are issued in up to this many pieces, spread over its row groups: eight wavefronts
+  // that issue their seven loads at once right after the barrier wait for the address unit, all
+  // together, before their first MFMA (T=4000 layer 413 -> 402 us, skewed T=4096 batch 1152 -> 1125,
+  // T=8192 608 -> 598, T=14107 940 -> 921; with weights hot in the L2s a K-step took as long
+  // as its loads alone and its MFMAs alone together). More pieces need more registers than the
+  // 160-row instances have (GEMM1 in three spills 4, GEMM2 in two 11: no faster).
+  constexpr int kMaxPieces = ROWS == kTileItemRowsMid ? 3 : G1 ? 2 : 1;
+  constexpr int kPieces = kMaxPieces < NG ? kMaxPieces : NG > 0 ? NG : 1;
+  auto compute = [&](int s, const Head& h, float s0, float s1, int kk, int sn) __attribute__((always_inline)) {
+    if constexpr (NG == 0) issue(kk, sn);
     if constexpr (NG > 0) {
       const TileStage<ROWS>& st = sh.st[s];
       const v8i (&wf)[4] = h.wf;
@@ -322,6 +338,13 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
       float sa = h.sa;
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
+        // a piece of the loads of step kk
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i)
+          if (g == i * NG / kPieces) {
+            issue_some(kk, sn, i * S::kLoadsPerStep / kPieces, (i + 1) * S::kLoadsPerStep / kPieces);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         // the next row group's fragment is read from LDS while this group's MFMAs run
         v8i bf_next = bf;
         float sa_next = sa;
@@ -354,7 +377,8 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // W32: per item group the four MFMAs (two weight blocks x two K halves) first, then their
   // scale promotion, acc += d_h * (s_act,h * s_w), in issue order, so that each FMA finds its
   // MFMA done; the next group's fragment and scales are read from LDS meanwhile.
-  auto compute32 = [&](int s, const Head32& h, float s0) __attribute__((always_inline)) {
+  auto compute32 = [&](int s, const Head32& h, float s0, int kk, int sn) __attribute__((always_inline)) {
+    if constexpr (NG == 0) issue(kk, sn);
     if constexpr (NG > 0) {
       const TileStage<ROWS>& st = sh.st[s];
       v8i bf[2] = {h.bf[0], h.bf[1]};
@@ -375,6 +399,9 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
         for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) d[blk][hh] = mfma32x32x64_fp8(h.wf[blk][hh], bf[hh], zero16);
+        __builtin_amdgcn_sched_barrier(0);
+        issue_some(kk, sn, g * S::kLoadsPerStep / NG, (g + 1) * S::kLoadsPerStep / NG);
+        __builtin_amdgcn_sched_barrier(0);
         const float q0 = sa[0] * s0, q1 = sa[1] * s0;
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
@@ -417,17 +444,13 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
       Head32 h;
       load_head32(s_cur, h);
       __builtin_amdgcn_sched_barrier(0);
-      issue(k + 2, s_next);
-      __builtin_amdgcn_sched_barrier(0);
-      compute32(s_cur, h, s0);
+      compute32(s_cur, h, s0, k + 2, s_next);
     } else {
       Head h;
       load_head(s_cur, h);
       __builtin_amdgcn_sched_barrier(0);
-      issue(k + 2, s_next);
-      __builtin_amdgcn_sched_barrier(0);
       const float s1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sw1_lane), k));
-      compute(s_cur, h, s0, s1);
+      compute(s_cur, h, s0, s1, k + 2, s_next);
     }
     s_cur = s_cur == kStages - 1 ? 0 : s_cur + 1;
     s_next = s_next == kStages - 1 ? 0 : s_next + 1;
