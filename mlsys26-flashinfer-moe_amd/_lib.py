@@ -120,11 +120,14 @@ class MoeFp8Layout(ctypes.Structure):
 
 _lock = threading.Lock()
 _lib = None
+_bytes_entries = None
 
 
 def load() -> ctypes.CDLL:
     """Loads libmoe_fp8.so once and declares the prototypes. Raises if it is not built."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -168,6 +171,20 @@ def load() -> ctypes.CDLL:
         lib.moe_fp8_version.restype = ctypes.c_char_p
         _lib = lib
         return lib
+
+
+def bytes_entries():
+    """moe_fp8_run and moe_fp8_run_packed with struct moe_fp8_args passed as a bytes object."""
+    global _bytes_entries
+    if _bytes_entries is None:
+        lib = load()
+        vp, sz = ctypes.c_void_p, ctypes.c_size_t
+        run, run_packed = lib["moe_fp8_run"], lib["moe_fp8_run_packed"]   # function objects of their own
+        run.argtypes = [ctypes.c_char_p, vp, sz, vp]
+        run_packed.argtypes = [ctypes.c_char_p, vp, sz, vp, sz, vp]
+        run.restype = run_packed.restype = ctypes.c_int
+        _bytes_entries = run, run_packed
+    return _bytes_entries
 
 
 def strerror(code: int) -> str:

@@ -7,6 +7,8 @@ places tensors on the GPU, manages the per-stream workspace and passes raw point
 """
 from __future__ import annotations
 
+import functools
+import struct
 import threading
 
 import torch
@@ -126,7 +128,9 @@ class WorkspaceCache:
         self._cache = {}
         self._retired = []
 
-    def get(self, key, num_tokens: int, need_bytes: int, device, stream):
+    def get(self, key, num_tokens: int, need_bytes: int, device, stream, capturing=None):
+        """The workspace of `key`, grown to need_bytes (capturing: whether the current stream is
+        being captured, where the caller knows)."""
         with self._lock:
             ws = self._cache.get(key)
             if ws is None or ws.buffer.numel() < need_bytes:
@@ -137,7 +141,7 @@ class WorkspaceCache:
             elif ws.layout.num_tokens != num_tokens:
                 ws.layout = _lib.workspace_layout(num_tokens)
                 ws.nbytes = int(ws.layout.total_bytes)
-            if self._capturing():
+            if self._capturing() if capturing is None else capturing:
                 ws.captured = True
             return ws
 
@@ -191,7 +195,7 @@ class PackedWeightCache:
         self._make = make or (lambda w13, w2: pack_weights(w13, w2))
         self._capturing = capturing or torch.cuda.is_current_stream_capturing
         self._ref = storage_ref or (lambda t: StorageWeakRef(t.untyped_storage()))
-        self._stream_id = stream_id or (lambda: torch.cuda.current_stream().cuda_stream)
+        self._stream_id = stream_id or _current_stream_id
         self._record = record or (lambda packed: packed.record_stream(torch.cuda.current_stream(packed.device)))
         self._event = event or _record_event
         self._wait = wait or (lambda ev: torch.cuda.current_stream().wait_event(ev))
@@ -200,15 +204,17 @@ class PackedWeightCache:
         self._retired = []
         self._failed = set()   # weight sets whose copy did not fit in device memory
 
-    def get(self, w13: torch.Tensor, w2: torch.Tensor):
+    def get(self, w13: torch.Tensor, w2: torch.Tensor, capturing=None):
         """The packed copy for (w13, w2), built if missing or stale; None when the set does
-        not fit or the stream is being captured without a copy."""
+        not fit or the stream is being captured without a copy (capturing: whether it is, where
+        the caller knows)."""
         if self.max_sets <= 0:
             return None
         key = (w13.device.index, w13.data_ptr(), w2.data_ptr())
         version = (w13._version, w2._version)
         with self._lock:
-            capturing = self._capturing()
+            if capturing is None:
+                capturing = self._capturing()
             stream = self._stream_id()
             ent = self._entries.get(key)
             if ent is not None and not ent["ref13"].expired() and not ent["ref2"].expired() \
@@ -255,6 +261,12 @@ class PackedWeightCache:
     @property
     def retired(self) -> list:
         return list(self._retired)
+
+
+def _current_stream_id() -> int:
+    """The current stream's handle on the current device (torch.cuda.current_stream().cuda_stream
+    without the stream object)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _record_event():
@@ -307,7 +319,70 @@ def make_args(routing_logits, routing_bias, hidden_states, hidden_states_scale, 
     return a
 
 
-@torch.no_grad()
+# struct moe_fp8_args as bytes (make_args without the ctypes object)
+_ARGS = struct.Struct("@PPiPPPPPPiifPi0P")
+_layer_bytes = functools.lru_cache(maxsize=4096)(_lib.workspace_bytes)
+
+
+def _run_direct(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
+                gemm2_weights, gemm2_weights_scale, local_expert_offset, routed_scaling_factor, output, packed) -> bool:
+    """The common call: every tensor on the current GPU, contiguous, aligned and of the contract's
+    type and shape, so that nothing is moved, copied or converted and no torch operation runs.
+    Returns False, having done nothing, for every other call: _run handles those (and raises
+    what there is to raise). With _run's general path a decode call of one token was bound by its
+    ~33 us of host time, the GPU's work taking 23."""
+    T = routing_logits.shape[0] if routing_logits.dim() == 2 else 0
+    bias_code = _BIAS_CODES.get(routing_bias.dtype)
+    f32, fp8 = torch.float32, torch.float8_e4m3fn
+    if T == 0 or bias_code is None or not (
+            hidden_states.dtype is fp8 and gemm1_weights.dtype is fp8 and gemm2_weights.dtype is fp8
+            and routing_logits.dtype is f32 and hidden_states_scale.dtype is f32
+            and gemm1_weights_scale.dtype is f32 and gemm2_weights_scale.dtype is f32
+            and (output.dtype is torch.bfloat16 or output.dtype is f32)):
+        return False
+    # (the contract puts no shape on the bias; what is not [256] takes the general path)
+    if not (routing_logits.shape[1] == EXPERTS_GLOBAL and routing_bias.shape == (EXPERTS_GLOBAL,)
+            and hidden_states.shape == (T, HIDDEN) and hidden_states_scale.shape == (H_BLOCKS, T)
+            and gemm1_weights.shape == (EXPERTS_LOCAL, 2 * INTER, HIDDEN)
+            and gemm1_weights_scale.shape == (EXPERTS_LOCAL, G1_BLOCKS, H_BLOCKS)
+            and gemm2_weights.shape == (EXPERTS_LOCAL, HIDDEN, INTER)
+            and gemm2_weights_scale.shape == (EXPERTS_LOCAL, H_BLOCKS, I_BLOCKS) and output.shape == (T, HIDDEN)):
+        return False
+    dev = output.get_device() if output.is_cuda else -1
+    if dev < 0 or torch._C._cuda_getDevice() != dev:
+        return False
+    ptrs = []
+    for t in (routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
+              gemm2_weights, gemm2_weights_scale, output):
+        if not t.is_cuda or t.get_device() != dev or not t.is_contiguous():
+            return False
+        ptrs.append(t.data_ptr())
+    logits, bias, hidden, hidden_scale, w13, w13_scale, w2, w2_scale, out = ptrs
+    if (logits | hidden | w13 | w2 | out) & 15 or (bias | hidden_scale | w13_scale | w2_scale) & 3:
+        return False
+    try:
+        args = _ARGS.pack(logits, bias, bias_code, hidden, hidden_scale, w13, w13_scale, w2, w2_scale, T,
+                          int(local_expert_offset), float(routed_scaling_factor), out,
+                          OUT_F32 if output.dtype is f32 else OUT_BF16)
+    except (OverflowError, struct.error):
+        return False   # a value that ctypes wraps or rounds
+    if packed is not None and packed is not _AUTO and packed.device != output.device:
+        return False
+    capturing = torch.cuda.is_current_stream_capturing()
+    stream = torch._C._cuda_getCurrentRawStream(dev)
+    ws = _workspaces.get((dev, stream), T, _layer_bytes(T), output.device, None, capturing)
+    if packed is _AUTO:
+        packed = _packed_weights.get(gemm1_weights, gemm2_weights, capturing) if T <= PACKED_MAX_TOKENS else None
+    run_args, run_packed_args = _lib.bytes_entries()
+    with ws.lock:
+        if packed is None:
+            _lib.check(run_args(args, ws.ptr, ws.buffer.numel(), stream), "moe_fp8_run")
+        else:
+            _lib.check(run_packed_args(args, packed.data_ptr(), packed.numel(), ws.ptr, ws.buffer.numel(), stream),
+                       "moe_fp8_run_packed")
+    return True
+
+
 def run(
     routing_logits: torch.Tensor,
     routing_bias: torch.Tensor,
@@ -333,8 +408,10 @@ def run(
     of the weight set that the first such call builds and later calls reuse (PackedWeightCache;
     set_packed_weight_sets(0) turns it off). The output is bit-identical either way.
     """
-    _run(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
-         gemm2_weights, gemm2_weights_scale, local_expert_offset, routed_scaling_factor, output, _AUTO)
+    args = (routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
+            gemm2_weights, gemm2_weights_scale, local_expert_offset, routed_scaling_factor, output, _AUTO)
+    if not _run_direct(*args):
+        _run(*args)
     return None
 
 
@@ -366,7 +443,6 @@ def pack_weights(gemm1_weights: torch.Tensor, gemm2_weights: torch.Tensor) -> to
     return packed
 
 
-@torch.no_grad()
 def run_packed(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights,
                gemm1_weights_scale, gemm2_weights, gemm2_weights_scale, local_expert_offset: int,
                routed_scaling_factor: float, output: torch.Tensor, *, packed_weights: torch.Tensor):
@@ -375,11 +451,14 @@ def run_packed(routing_logits, routing_bias, hidden_states, hidden_states_scale,
     to run()'s."""
     assert packed_weights.dtype == torch.uint8 and packed_weights.is_contiguous() and \
         packed_weights.numel() >= _lib.packed_weights_bytes(), "packed_weights must come from pack_weights"
-    _run(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
-         gemm2_weights, gemm2_weights_scale, local_expert_offset, routed_scaling_factor, output, packed_weights)
+    args = (routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
+            gemm2_weights, gemm2_weights_scale, local_expert_offset, routed_scaling_factor, output, packed_weights)
+    if not _run_direct(*args):
+        _run(*args)
     return None
 
 
+@torch.no_grad()
 def _run(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
          gemm2_weights, gemm2_weights_scale, local_expert_offset, routed_scaling_factor, output, packed):
     T = validate(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights,
@@ -430,7 +509,27 @@ def _run(routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1
 _HIDDEN_CODES = {torch.float32: HIDDEN_F32, torch.bfloat16: HIDDEN_BF16, torch.float16: HIDDEN_F16}
 
 
-@torch.no_grad()
+def _quantize_direct(x, out, out_scale) -> bool:
+    """quantize_hidden's common call: everything on the current GPU, contiguous, aligned, of the
+    contract's type and shape. Returns False, having done nothing, for every other call."""
+    code = _HIDDEN_CODES.get(x.dtype)
+    if code is None or not x.is_cuda or x.dim() != 2 or out is None or out_scale is None:
+        return False
+    T, dev = x.shape[0], x.get_device()
+    if not (T > 0 and x.shape[1] == HIDDEN and x.is_contiguous() and torch._C._cuda_getDevice() == dev
+            and out.dtype is torch.float8_e4m3fn and out.shape == (T, HIDDEN) and out.is_cuda
+            and out.get_device() == dev and out.is_contiguous()
+            and out_scale.dtype is torch.float32 and out_scale.shape == (H_BLOCKS, T) and out_scale.is_cuda
+            and out_scale.get_device() == dev and out_scale.is_contiguous()):
+        return False
+    px, pq, ps = x.data_ptr(), out.data_ptr(), out_scale.data_ptr()
+    if px & 15 or pq & 7 or ps & 3:
+        return False
+    _lib.check(_lib.load().moe_fp8_quantize_hidden(px, code, T, pq, ps, torch._C._cuda_getCurrentRawStream(dev)),
+               "moe_fp8_quantize_hidden")
+    return True
+
+
 def quantize_hidden(hidden: torch.Tensor, out: torch.Tensor | None = None,
                     out_scale: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """The step before `run`: hidden states [T, 7168] (bf16, fp16 or fp32) to the layer's
@@ -441,6 +540,13 @@ def quantize_hidden(hidden: torch.Tensor, out: torch.Tensor | None = None,
     Returns (hidden_states, hidden_states_scale), written into `out` / `out_scale` when
     given (contiguous tensors of those shapes and dtypes on the input's GPU).
     """
+    if _quantize_direct(hidden, out, out_scale):
+        return out, out_scale
+    return _quantize(hidden, out, out_scale)
+
+
+@torch.no_grad()
+def _quantize(hidden, out, out_scale):
     assert hidden.dtype in _HIDDEN_CODES, "hidden must be float32, bfloat16 or float16"
     assert hidden.dim() == 2 and hidden.shape[1] == HIDDEN, "hidden must be [T, 7168]"
     device = _ensure_cuda(hidden, out, out_scale)
