@@ -52,7 +52,8 @@
 //          knows the next one in time to prefetch its first K-steps. Measured against
 //          contiguous blocks of units per XCD: GEMM1 296 against 313 us at T=8192, 164
 //          against 174 at T=1024, 656 against 682 on the skewed T=4096 batch; GEMM2 +
-//          combine 114 against 123 us at T=1024.
+//          combine 114 against 123 us at T=1024. GEMM1 with 128-row items splits the units of a
+//          sparse last round into halves of 64 columns (XcdList::split_tail).
 //   Work runs with stealing (GEMM2 with items of up to 160 rows): XCD x owns a contiguous run
 //          of the unit numbering, cut at weight-tile boundaries where the estimated work (item
 //          rows plus a fixed cost per unit) reaches x/8 and (x+1)/8 of the launch's; its
@@ -175,6 +176,7 @@ struct TileCtx {
   float sw0_lane, sw1_lane;     // lane k: weight block scale of K-step k of fragments 0,1
                                // (GEMM1 gate) and 2,3 (GEMM1 up)
   int r0, rows, tile, m0;      // item rows [r0, r0+rows); first item row of this wave's half
+  int half;                    // GEMM1: the 64-column half of the tile, or -1 for the whole tile
   int ng;                      // row groups of this wave's half
   // GEMM2: the destination (token, or -1 - flat slot) and routing weight of the lane's row in
   // each of this wave's row groups, loaded when the unit is set up (a unit ahead) so that the
@@ -202,7 +204,9 @@ __device__ __forceinline__ v8i lds_frag32(const uint8_t* buf, int m, int hh, int
 // unit (n) when `have_n`, and `pre` says that this unit's were loaded so. GEMM1 (56 K-steps)
 // does not (the per-step address selects cost it more than the saved ring fill): its last two
 // steps, like GEMM2's last unit's, load the last step again into stages nobody reads.
-template <bool G1, int NG, int ROWS>
+// WF: weight fragments per wavefront, 4 for a whole tile, 2 for a half (GEMM1: 64 SwiGLU columns, tile
+// rows 0..63 their gate rows and 64..127 their up rows, 16 columns per wavefront).
+template <bool G1, int NG, int ROWS, int WF>
 __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROWS>& c, const TileCtx<ROWS>& n,
                                           bool have_n, int s_base, bool pre, TileShared<ROWS>& sh,
                                           unsigned long long* claim, unsigned long long inc) {
@@ -211,6 +215,9 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // GEMM2 with two activation scales per K-step (64-column requantisation blocks): 32x32x64
   // MFMAs, NG counts 32-row item groups
   constexpr bool W32 = !G1 && S::kW32;
+  constexpr int kWLoads = kWDma * WF / 4;             // weight DMA loads per wavefront per step
+  constexpr int kLoads = kWLoads + S::kLoadsPerStep - kWDma;
+  static_assert(WF == 4 || (WF == 2 && G1 && S::kQCols == 64), "half tiles: GEMM1 with 64-column blocks");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wb = wave & 3;     // weight rows 64*wb.. (item rows: the wave's half, from c.m0)
@@ -226,20 +233,20 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // select of the source addresses, so the loop has no branch. Every lane loads (activation
   // rows and scale rows past the item's end repeat its first row into slots nobody reads), so
   // no load is divergent; every wave loads even if it has no rows.
-  // Loads [from, to) of the step's S::kLoadsPerStep.
+  // Loads [from, to) of the step's kLoads.
   auto issue_some = [&](int kk, int s, int from, int to) __attribute__((always_inline)) {
     const bool nxt = !G1 && kk >= KS && have_n;
     const int k = kk < KS ? kk : (nxt ? kk - KS : KS - 1);
     TileStage<ROWS>& st = sh.st[s];
     const uint8_t* wk = (nxt ? n.wbase : c.wbase) + k * 128;
 #pragma unroll
-    for (int j = 0; j < kWDma; ++j)
-      if (from <= j && j < to) dma16(wk + (nxt ? n.woff[j] : c.woff[j]), &st.w[(32 * wave + 8 * j) * 128]);
+    for (int j = 0; j < kWLoads; ++j)
+      if (from <= j && j < to) dma16(wk + (nxt ? n.woff[j] : c.woff[j]), &st.w[(8 * kWLoads * wave + 8 * j) * 128]);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      if (from <= kWDma + j && kWDma + j < to)
+      if (from <= kWLoads + j && kWLoads + j < to)
         dma16((nxt ? n.asrc[j] : c.asrc[j]) + k * 128, &st.a[8 * (wave + kTileWaves * j) * 128]);
-    if (from <= kWDma + 2 && kWDma + 2 < to) {
+    if (from <= kWLoads + 2 && kWLoads + 2 < to) {
       const float* sk = (nxt ? n.ssrc : c.ssrc) + k * c.sstride;
       if constexpr (S::kThirdBlock) {
         if (wave < 4) dma16((nxt ? n.asrc[2] : c.asrc[2]) + k * 128, &st.a[8 * (wave + 2 * kTileWaves) * 128]);
@@ -249,10 +256,10 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
       }
     }
   };
-  auto issue = [&](int kk, int s) __attribute__((always_inline)) { issue_some(kk, s, 0, S::kLoadsPerStep); };
+  auto issue = [&](int kk, int s) __attribute__((always_inline)) { issue_some(kk, s, 0, kLoads); };
 
   constexpr int NG1 = NG > 0 ? NG : 1;
-  v4f acc[W32 ? 1 : 4][W32 ? 1 : NG1];
+  v4f acc[W32 ? 1 : WF][W32 ? 1 : NG1];
   v16f acc32[W32 ? 2 : 1][W32 ? NG1 : 1];   // W32: [weight rows 32*blk..][item group]
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
   const v16f zero16 = {};
@@ -263,15 +270,17 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
       for (int g = 0; g < NG; ++g) acc32[blk][g] = zero16;
   } else {
 #pragma unroll
-    for (int f = 0; f < 4; ++f)
+    for (int f = 0; f < WF; ++f)
 #pragma unroll
       for (int g = 0; g < NG; ++g) acc[f][g] = zero;
   }
 
   // weight fragment f of this wave: GEMM1 gate rows 32*wb + 16f (f = 0,1) and the up rows
-  // 128 + 32*wb + 16(f-2) (f = 2,3); GEMM2 rows 64*wb + 16f
+  // 128 + 32*wb + 16(f-2) (f = 2,3), or of a half tile gate rows 16*wb (f = 0) and up rows 64 + 16*wb
+  // (f = 1); GEMM2 rows 64*wb + 16f
   auto wrow = [&](int f) {
-    if constexpr (G1) return (f < 2 ? 32 * wb + 16 * f : 128 + 32 * wb + 16 * (f - 2)) + (lane & 15);
+    if constexpr (WF == 2) return 64 * f + 16 * wb + (lane & 15);
+    else if constexpr (G1) return (f < 2 ? 32 * wb + 16 * f : 128 + 32 * wb + 16 * (f - 2)) + (lane & 15);
     else return 64 * wb + 16 * f + (lane & 15);
   };
 
@@ -279,7 +288,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // They are read from LDS right after the barrier, before the step's DMA issue, so that
   // the issue overlaps their latency.
   struct Head {
-    v8i wf[4];
+    v8i wf[WF];
     v8i bf;
     float sa;
   };
@@ -289,7 +298,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
       h.bf = lds_frag(st.a + c.m0 * 128, lane & 15, lane);
       h.sa = st.sa[c.m0 + (lane & 15)];
 #pragma unroll
-      for (int f = 0; f < 4; ++f) h.wf[f] = lds_frag(st.w, wrow(f), lane);
+      for (int f = 0; f < WF; ++f) h.wf[f] = lds_frag(st.w, wrow(f), lane);
     }
   };
   // W32: the wave's two 32-row weight blocks and its first item group, each as two 64-wide
@@ -318,7 +327,9 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // and accumulated while the MFMAs of the next group run (the last group of a K-step while
   // the first group of the next step runs), so that the matrix core is not idle during the
   // VALU work. dp holds the pending group's MFMA results, p0/p1 its two scale products.
-  v4f dp[4] = {zero, zero, zero, zero};
+  v4f dp[WF];
+#pragma unroll
+  for (int f = 0; f < WF; ++f) dp[f] = zero;
   float p0 = 0.f, p1 = 0.f;
 
   // A step's loads are issued in up to this many pieces, spread over its row groups: eight wavefronts
@@ -333,7 +344,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
     if constexpr (NG == 0) issue(kk, sn);
     if constexpr (NG > 0) {
       const TileStage<ROWS>& st = sh.st[s];
-      const v8i (&wf)[4] = h.wf;
+      const v8i (&wf)[WF] = h.wf;
       v8i bf = h.bf;
       float sa = h.sa;
 #pragma unroll
@@ -342,7 +353,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
 #pragma unroll
         for (int i = 0; i < kPieces; ++i)
           if (g == i * NG / kPieces) {
-            issue_some(kk, sn, i * S::kLoadsPerStep / kPieces, (i + 1) * S::kLoadsPerStep / kPieces);
+            issue_some(kk, sn, i * kLoads / kPieces, (i + 1) * kLoads / kPieces);
             __builtin_amdgcn_sched_barrier(0);
           }
         // the next row group's fragment is read from LDS while this group's MFMAs run
@@ -355,14 +366,14 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
         // pending group: the previous group of this step, or the previous step's last
         // group (zero results and zero scales before the first step)
         const int gp = g == 0 ? NG - 1 : g - 1;
-        v4f d[4];
+        v4f d[WF];
 #pragma unroll
-        for (int f = 0; f < 4; ++f) {
+        for (int f = 0; f < WF; ++f) {
           d[f] = mfma16x16x128_fp8(wf[f], bf, zero);
-          acc[f][gp] += dp[f] * (f < 2 ? p0 : p1);
+          acc[f][gp] += dp[f] * (f < WF / 2 ? p0 : p1);
         }
 #pragma unroll
-        for (int f = 0; f < 4; ++f) dp[f] = d[f];
+        for (int f = 0; f < WF; ++f) dp[f] = d[f];
         p0 = sa * s0;
         p1 = sa * s1;
         // two row groups' MFMA results live at a time (the scheduler would otherwise hoist
@@ -400,7 +411,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) d[blk][hh] = mfma32x32x64_fp8(h.wf[blk][hh], bf[hh], zero16);
         __builtin_amdgcn_sched_barrier(0);
-        issue_some(kk, sn, g * S::kLoadsPerStep / NG, (g + 1) * S::kLoadsPerStep / NG);
+        issue_some(kk, sn, g * kLoads / NG, (g + 1) * kLoads / NG);
         __builtin_amdgcn_sched_barrier(0);
         const float q0 = sa[0] * s0, q1 = sa[1] * s0;
 #pragma unroll
@@ -435,7 +446,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
     // A prefetched unit's first two steps landed before the previous unit's epilogue stored
     // anything (below): those steps do not wait, so the stores drain under their MFMAs (the
     // counter is in order, a wait for a later load waits for them).
-    if (!pre || k >= 2) wait_vmcnt<S::kLoadsPerStep>();
+    if (!pre || k >= 2) wait_vmcnt<kLoads>();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -458,7 +469,7 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
   // the last step's last row group
   if constexpr (NG > 0 && !W32) {
 #pragma unroll
-    for (int f = 0; f < 4; ++f) acc[f][NG - 1] += dp[f] * (f < 2 ? p0 : p1);
+    for (int f = 0; f < WF; ++f) acc[f][NG - 1] += dp[f] * (f < WF / 2 ? p0 : p1);
   }
   // The loads in flight now are the next unit's first two steps, or reloads nobody reads; the
   // reloads must land before the next unit refills the ring.
@@ -479,15 +490,17 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    float cval[NG > 0 ? NG : 1][2][4];
+    constexpr int kCols = WF / 2;                       // 16-column runs per wavefront
+    const int col0 = c.tile * 128 + (WF == 4 ? 32 * wb : 64 * c.half + 16 * wb);
+    float cval[NG > 0 ? NG : 1][kCols][4];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       float amax = 0.f;
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < kCols; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float x1 = acc[h][g][i], x2 = acc[2 + h][g][i];
+          const float x1 = acc[h][g][i], x2 = acc[kCols + h][g][i];
           cval[g][h][i] = x2 * __builtin_amdgcn_rcpf(1.0f + __expf(-x2)) * x1;
           amax = fmaxf(amax, fabsf(cval[g][h][i]));
         }
@@ -499,20 +512,20 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const int m = c.m0 + 16 * g + (lane & 15);
-      const float amax = S::kQCols == 64
+      const float amax = S::kQCols == 64 && WF == 4
                              ? fmaxf(amax_buf[wb & 2][m], amax_buf[(wb & 2) + 1][m])
                              : fmaxf(fmaxf(amax_buf[0][m], amax_buf[1][m]), fmaxf(amax_buf[2][m], amax_buf[3][m]));
       const float scale = fmaxf(amax / 448.0f, 1e-12f);
       const float inv = __builtin_amdgcn_rcpf(scale);
       if (m < c.rows) {
-        uint8_t* dst = p.act + (size_t)(c.r0 + m) * kInter + c.tile * 128 + 32 * wb + 4 * (lane >> 4);
+        uint8_t* dst = p.act + (size_t)(c.r0 + m) * kInter + col0 + 4 * (lane >> 4);
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < kCols; ++h)
           *reinterpret_cast<uint32_t*>(dst + 16 * h) =
               pack_fp8x4(cval[g][h][0] * inv, cval[g][h][1] * inv, cval[g][h][2] * inv, cval[g][h][3] * inv);
         // the first wave of each scale block writes the block's scale
-        if ((wb & (S::kQCols / 32 - 1)) == 0 && lane < 16)
-          p.act_scale[(size_t)(c.r0 + m) * S::kQBlocks + (c.tile * 128 + 32 * wb) / S::kQCols] = scale;
+        if ((wb & (S::kQCols / (16 * kCols) - 1)) == 0 && lane < 16)
+          p.act_scale[(size_t)(c.r0 + m) * S::kQBlocks + col0 / S::kQCols] = scale;
       }
     }
     __syncthreads();
@@ -570,16 +583,16 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
 }
 
 // NG (row groups of this wave's half) as a template argument: instantiations 0..kMaxNG.
-template <bool G1, int ROWS, int NG = 0>
+template <bool G1, int ROWS, int WF = 4, int NG = 0>
 __device__ __forceinline__ void tile_body_ng(const GemmParams& p, const TileCtx<ROWS>& c, const TileCtx<ROWS>& n,
                                              bool have_n, int s_base, bool pre, TileShared<ROWS>& sh,
                                              unsigned long long* claim, unsigned long long inc) {
   constexpr int kMax = (!G1 && TileShape<ROWS>::kW32) ? TileShape<ROWS>::kMaxNG32 : TileShape<ROWS>::kMaxNG;
   if constexpr (NG < kMax) {
-    if (c.ng == NG) tile_body<G1, NG, ROWS>(p, c, n, have_n, s_base, pre, sh, claim, inc);
-    else tile_body_ng<G1, ROWS, NG + 1>(p, c, n, have_n, s_base, pre, sh, claim, inc);
+    if (c.ng == NG) tile_body<G1, NG, ROWS, WF>(p, c, n, have_n, s_base, pre, sh, claim, inc);
+    else tile_body_ng<G1, ROWS, WF, NG + 1>(p, c, n, have_n, s_base, pre, sh, claim, inc);
   } else {
-    tile_body<G1, NG, ROWS>(p, c, n, have_n, s_base, pre, sh, claim, inc);
+    tile_body<G1, NG, ROWS, WF>(p, c, n, have_n, s_base, pre, sh, claim, inc);
   }
 }
 
@@ -607,12 +620,21 @@ __device__ __forceinline__ ExpertTable expert_table(const GemmParams& p, int n_i
   return t;
 }
 
+// A list entry: the work unit, and above kHalfShift 1 or 2 for one of its halves (kSplitTail).
+constexpr int kHalfShift = 28;
+constexpr int kUnitMask = (1 << kHalfShift) - 1;
+// GEMM1 with 128-row items splits the units of a sparse last round into halves.
+template <bool G1, int ROWS>
+constexpr bool kSplitTail = G1 && ROWS == kTileItemRowsMid;
+
 // The pointers and item of work unit u for this lane (all of it wave-uniform but the DMA
 // offsets and the lane's block scales). Unit u of the expert whose items start at item `first`
 // is (item first + v % items, weight tile v / items) with v = u - first * TILES.
 template <bool G1, int ROWS>
-__device__ __forceinline__ void unit_setup(const GemmParams& p, const ExpertTable& tab, int u, TileCtx<ROWS>& c) {
+__device__ __forceinline__ void unit_setup(const GemmParams& p, const ExpertTable& tab, int entry, TileCtx<ROWS>& c) {
   using S = TileShape<ROWS>;
+  const int u = entry & kUnitMask;
+  c.half = (entry >> kHalfShift) - 1;
   constexpr int TILES = (G1 ? 2 * kInter : kHidden) / kTileW;
   constexpr int KS = G1 ? kHBlocks : kIBlocks;
   const int lane = threadIdx.x & 63;
@@ -636,10 +658,13 @@ __device__ __forceinline__ void unit_setup(const GemmParams& p, const ExpertTabl
   // (activation rows past the item's end repeat its first row)
 #pragma unroll
   for (int j = 0; j < kWDma; ++j) {
-    const int r = 32 * wave + 8 * j + (lane >> 3);
+    // (a half tile: 16 rows per wave, loads j = 0 and 1)
+    const bool half = kSplitTail<G1, ROWS> && c.half >= 0;
+    const int r = (half ? 16 : 32) * wave + 8 * j + (lane >> 3);
     const int ch = (lane & 7) ^ ((r >> 1) & 7);
     size_t grow;
-    if constexpr (G1) grow = (size_t)e * 2 * kInter + (r < 128 ? c.tile * 128 + r : kInter + c.tile * 128 + r - 128);
+    if (half) grow = (size_t)e * 2 * kInter + ((r & 64) ? kInter : 0) + c.tile * 128 + 64 * c.half + (r & 63);
+    else if constexpr (G1) grow = (size_t)e * 2 * kInter + (r < 128 ? c.tile * 128 + r : kInter + c.tile * 128 + r - 128);
     else grow = (size_t)e * kHidden + c.tile * kTileW + r;
     c.woff[j] = (uint32_t)(grow * (G1 ? kHidden : kInter) + ch * 16);
   }
@@ -705,11 +730,33 @@ template <int TILES>
 struct XcdList {
   int first, ne, t0, pos;
   int total;   // entries of the list (wave-uniform)
+  int whole;   // entries before the half tiles (split_tail; all of them without)
+
+  // The list's units fill the XCD's work-groups in rounds. When the last round would hold at most
+  // half of them, its units are split into halves (64 columns each) for the idle ones: such a round
+  // is bound by what one CU can stream alone (~50 GB/s from HBM however deep its ring, a unit of
+  // 1.8 MB 44-48 us), and a half takes half as long. In a fuller round the CUs share the HBM's
+  // rate and halves only double the activation loads. Whole layer, whole / split: T=300 with 21
+  // items (10 units over) 211 / 201 us, T=512 with 20 (8 over) 205 / 195, T=901 with 22 (12 over)
+  // 222 / 215, T=2048 with 33 (2 over) 329 / 318, T=512 with 24 (16 over, the most that are split)
+  // 221 / 216. Bit-identical.
+  __device__ __forceinline__ void split_tail(int work_groups) {
+    const int r = total % work_groups;
+    if (2 * r <= work_groups) {
+      whole = total - r;
+      total += r;
+    }
+  }
 
   // Work unit of list entry j; false past the end. j must be wave-uniform.
   __device__ __forceinline__ bool entry(int j, int& u) const {
     if (j >= total) return false;
     const int lane = threadIdx.x & 63;
+    int half = 0;   // 1, 2: a half tile
+    if (j >= whole) {
+      half = 1 + ((j - whole) & 1);
+      j = whole + ((j - whole) >> 1);
+    }
     // the last expert that starts at or before j (experts with units come first)
     const unsigned long long m = __ballot(lane < kExpertsLocal && ne > 0 && pos <= j);
     const int k = 63 - __builtin_clzll(m);
@@ -719,7 +766,7 @@ struct XcdList {
     const int ntx = (TILES - t0k + 7) >> 3;   // the expert's tiles on this XCD
     const int item = r / ntx;
     const int tile = t0k + 8 * (r - item * ntx);
-    u = __builtin_amdgcn_readlane(first, k) * TILES + tile * ne_k + item;
+    u = (__builtin_amdgcn_readlane(first, k) * TILES + tile * ne_k + item) | (half << kHalfShift);
     return true;
   }
 };
@@ -740,6 +787,7 @@ __device__ __forceinline__ XcdList<TILES> xcd_list(const ExpertTable& tab, int x
   }
   l.pos = incl - len;
   l.total = __builtin_amdgcn_readfirstlane(__shfl(incl, kExpertsLocal - 1));
+  l.whole = l.total;
   return l;
 }
 
@@ -930,8 +978,13 @@ __global__ __launch_bounds__(kTileWaves * 64, 1) void gemm_tile_kernel(GemmParam
       for (;;) {
         // GEMM2 claims the entry after the reserved one only while there is one
         const bool claim_now = G1 || have_n;
-        tile_body_ng<G1, ROWS>(p, c, n, have_n, s_base, pre_loaded, sh, claim_now ? claims + src : nullptr,
-                               src == x ? 1ull : 1ull << 32);
+        unsigned long long* const claim = claim_now ? claims + src : nullptr;
+        const unsigned long long inc = src == x ? 1ull : 1ull << 32;
+        if (kSplitTail<G1, ROWS> && c.half >= 0) {
+          if constexpr (kSplitTail<G1, ROWS>) tile_body_ng<G1, ROWS, 2>(p, c, n, have_n, s_base, pre_loaded, sh, claim, inc);
+        } else {
+          tile_body_ng<G1, ROWS>(p, c, n, have_n, s_base, pre_loaded, sh, claim, inc);
+        }
         // publishes sh.next (LDS); the unit's global stores may still be in flight
         wait_lgkmcnt0();
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -966,7 +1019,9 @@ __global__ __launch_bounds__(kTileWaves * 64, 1) void gemm_tile_kernel(GemmParam
     const RangeSet ranges = range_set<TILES>(tab, n_items);
     run_list(RangeList{ranges.begin_of(x), ranges.total_of(x)}, ranges);
   } else {
-    run_list(xcd_list<TILES>(tab, x), RangeSet{0, 0});
+    XcdList<TILES> list = xcd_list<TILES>(tab, x);
+    if constexpr (kSplitTail<G1, ROWS>) list.split_tail(per_xcd);
+    run_list(list, RangeSet{0, 0});
   }
 }
 
