@@ -225,8 +225,11 @@ int run_layer(const moe_fp8_args* args, void* workspace, size_t workspace_bytes,
   if (!mark(0)) return MOE_FP8_ELAUNCH;
   if (args->num_tokens <= kFusedDispatchTokens) {
     // routing, then GEMM1 with the dispatch rebuilt in every work-group: one launch less
-    if (launch_route(rp, stream) != hipSuccess || !mark(1)) return MOE_FP8_ELAUNCH;
-    if (launch_gemm1_dispatch(gp, rp, use_packed, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
+    // (the smallest batches are routed there too, unless routing is timed as a stage)
+    const bool route = !events && gemm1_dispatch_routes(args->num_tokens);
+    if (!route && launch_route(rp, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
+    if (!mark(1)) return MOE_FP8_ELAUNCH;
+    if (launch_gemm1_dispatch(gp, rp, use_packed, route, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
   } else {
     if (launch_route_dispatch(rp, stream) != hipSuccess || !mark(1)) return MOE_FP8_ELAUNCH;
     if (launch_gemm1(gp, L.rows_per_item, use_packed, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
