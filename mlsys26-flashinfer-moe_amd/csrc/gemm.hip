@@ -281,25 +281,26 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 
 __device__ __forceinline__ int lds_swz(int m, int c) { return m * 128 + ((c ^ ((m >> 1) & 7)) << 4); }
 
-// vmcnt(n) with expcnt and lgkmcnt left unconstrained (gfx9 s_waitcnt encoding).
+// vmcnt(n) with expcnt and lgkmcnt left unconstrained (gfx9 s_waitcnt encoding: vmcnt in bits
+// 3:0 and 15:14).
 template <int N>
 __device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 16, "vmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(N | (7 << 4) | (15 << 8));
+  static_assert(N >= 0 && N < 64, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
-template <int NG>
+// NB: ring slots (NB - 1 K-steps in flight besides the one consumed).
+template <int NG, int NB>
 __device__ __forceinline__ void stream_accumulate_g1_lds(const GemmParams& p, int e, int r0, int rows, int slice,
                                                          int lane, const int32_t* row_token, uint8_t* ring,
                                                          v4f (&acc)[2][NG]) {
   using S = StreamShape<kG1>;
   constexpr int KS = S::kSteps;
-  constexpr int NB = S::kRing;
   constexpr int KMAIN = KS - KS % NB;
   // VMEM instructions of one K-step, in issue order: the weight DMAs, then per row group the
   // activation fragment (two 16-byte loads) and its scale
   constexpr int kOps = kG1LdsDma + 3 * NG;
-  static_assert(kOps < 16, "vmcnt immediate");
+  static_assert(kOps * (NB - 1) < 64, "vmcnt immediate");
 
   // lane's DMA source of instruction j at K-step 0: ring row 8j + lane/8 (gate rows 0-15,
   // up rows 16-31), the logical chunk stored at physical chunk lane%8
@@ -361,8 +362,8 @@ __device__ __forceinline__ void stream_accumulate_g1_lds(const GemmParams& p, in
     issue_w(kn, sn);
     issue_a(kn, ring_a[sn]);
     __builtin_amdgcn_sched_barrier(0);
-    // step k's loads have landed once only step kn's are in flight
-    wait_vm<kOps>();
+    // step k's loads have landed once only those of the NB - 1 steps after it are in flight
+    wait_vm<kOps * (NB - 1)>();
     __builtin_amdgcn_sched_barrier(0);
     const uint8_t* st = ring + u * kG1LdsStep;
     v8i wf[2];
@@ -408,13 +409,15 @@ __device__ __forceinline__ v4f swiglu4(const v4f& x1, const v4f& x2) {
 // One work unit with its epilogue: GEMM1 writes fp32 SwiGLU rows for requant_kernel; GEMM2
 // writes or parks the weighted rows.
 // GEMM1 on row-major weights streams them through the wavefront's LDS ring `ring`
-// (kNB * kG1LdsStep bytes); the other instances do not use it.
+// (RING or StreamShape's kRing slots of kG1LdsStep bytes); the other instances do not use it.
 template <int KIND, int NG, bool PACKED = false, int RING = 0>
 __device__ __forceinline__ void stream_unit(const GemmParams& p, int e, int r0, int rows, int slice, int lane,
                                             const int32_t* row_token, uint8_t* ring) {
   constexpr int NF = StreamShape<KIND>::kFrags;
   v4f acc[NF][NG];
-  if constexpr (KIND == kG1 && !PACKED) stream_accumulate_g1_lds<NG>(p, e, r0, rows, slice, lane, row_token, ring, acc);
+  constexpr int kLdsSlots = RING > 0 ? RING : StreamShape<kG1>::kRing;
+  if constexpr (KIND == kG1 && !PACKED)
+    stream_accumulate_g1_lds<NG, kLdsSlots>(p, e, r0, rows, slice, lane, row_token, ring, acc);
   else stream_accumulate<KIND, NG, PACKED, RING>(p, e, r0, rows, slice, lane, row_token, acc);
   // lane: column (lane & 15) of each row group, fragment rows 4*(lane>>4) + i
 #pragma unroll
@@ -500,9 +503,10 @@ static_assert(kFusedHalves == 2, "two slots per thread");
 
 // The row-major instance's LDS weight rings live in the same object as the dispatch (one
 // __shared__ object: the compiler then keeps the ring's DMA writes apart from its reads).
-template <bool RING>
+// SLOTS: ring slots per wavefront, 0 without rings.
+template <int SLOTS>
 struct FusedDispatch {
-  uint8_t ring[RING ? kStreamWaves : 0][StreamShape<kG1>::kRing * kG1LdsStep];
+  uint8_t ring[SLOTS > 0 ? kStreamWaves : 0][SLOTS * kG1LdsStep];
   int4 items[kFusedItems];
   int32_t row_token[kFusedSlots];
   int cnt[kFusedHalves * kStreamWaves][kExpertsLocal];   // per-wavefront counts -> prefix
@@ -542,9 +546,9 @@ __device__ __forceinline__ void inline_route(const RouteParams& rp, InlineRoute&
 }
 
 // ids, weights: the top-k lists (the workspace's, or the work-group's own).
-template <bool RING>
+template <int SLOTS>
 __device__ __forceinline__ void fused_dispatch(const GemmParams& p, const RouteParams& rp, const int32_t* ids,
-                                               const float* weights, FusedDispatch<RING>& s) {
+                                               const float* weights, FusedDispatch<SLOTS>& s) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -640,17 +644,20 @@ __device__ __forceinline__ void fused_dispatch(const GemmParams& p, const RouteP
   __syncthreads();
 }
 
-// PACKED: p.w13 is the packed copy of W13 (moe_fp8_run_packed). RING: the depth of the packed
-// instance's register ring (0: StreamShape<kG1>::kRing; gemm1_stream_dispatch_deep_kernel).
+// PACKED: p.w13 is the packed copy of W13 (moe_fp8_run_packed). RING: the ring's depth (0:
+// StreamShape<kG1>::kRing; gemm1_stream_dispatch_deep_kernel); packed weights stream through
+// registers, row-major ones through LDS (4 KB per slot and wavefront).
 // Small batches take deeper rings (RING - 1 K-steps in flight per wavefront instead of one):
 // they touch a few experts, so only a few hundred wavefronts stream and each one's depth sets
 // the rate. Measured through the C ABI on seeded batches (two runs each, us per layer, 2 / 3 /
-// 4 slots): T=1 with 2 experts 34.6 / 30.8 / 29.3, T=2 with 3 experts 41.2 / 37.5 / 35.8, T=4
+// 4 slots, packed): T=1 with 2 experts 34.6 / 30.8 / 29.3, T=2 with 3 experts 41.2 / 37.5 / 35.8, T=4
 // with 4 experts 45.0 / 42.1 / 42.5, T=8 with 3 experts 41.6 / 37.7 / 36.2; with 5-6 experts
 // (640-768 units) within +-0.5; at T=16 (10 experts, 1280 units) 84.8 / 86.3 / 85.3, hence
 // the bound of 8 tokens. 4 / 6 / 8 slots: 2 experts (256 units) 30.4 / 28.4 / 28.0 and 30.3 /
 // 27.9 / 27.9, 3 experts 36.3 / 35.9 / 36.5, 5 experts 49.9 / 50.8 / 51.7: 6 slots up to 2
-// tokens. Bit-identical to the 2-slot ring.
+// tokens. The same depths on the row-major weights, 2 slots -> these: T=1 40.9 -> 35.8, T=2 44.5 ->
+// 40.8, T=3 47.8 -> 46.1, T=4 53.0 -> 50.9, T=5 55.0 -> 54.4, T=6 and T=8 within 0.4.
+// Bit-identical to the 2-slot ring.
 constexpr int kDeepRingTokens = 8;
 constexpr int kDeepRing = 4;
 constexpr int kDeeperRingTokens = 2;
@@ -659,13 +666,13 @@ constexpr int kDeeperRing = 6;
 // ROUTE: the kernel routes the batch itself (inline_route).
 template <bool PACKED, int RING, bool ROUTE>
 __device__ __forceinline__ void gemm1_stream_dispatch(const GemmParams& p, const RouteParams& rp) {
-  static_assert(RING == 0 || PACKED, "the row-major instance's LDS ring waits assume StreamShape's depth");
+  constexpr int kSlots = PACKED ? 0 : RING > 0 ? RING : StreamShape<kG1>::kRing;
   struct Shared {
-    FusedDispatch<!PACKED> d;
+    FusedDispatch<kSlots> d;
     InlineRoute r[ROUTE ? 1 : 0];
   };
   __shared__ __attribute__((aligned(1024))) Shared sh;
-  FusedDispatch<!PACKED>& s = sh.d;
+  FusedDispatch<kSlots>& s = sh.d;
   if constexpr (ROUTE) {
     inline_route(rp, sh.r[0]);
     fused_dispatch(p, rp, sh.r[0].ids, sh.r[0].w, s);
@@ -677,15 +684,15 @@ __device__ __forceinline__ void gemm1_stream_dispatch(const GemmParams& p, const
   stream_units<kG1, 1, PACKED, RING>(p, s.n_items, s.items, s.row_token, ring);
 }
 
-template <bool PACKED, bool ROUTE = false>
+template <bool PACKED>
 __global__ __launch_bounds__(kStreamWaves * 64) void gemm1_stream_dispatch_kernel(GemmParams p, RouteParams rp) {
-  gemm1_stream_dispatch<PACKED, 0, ROUTE>(p, rp);
+  gemm1_stream_dispatch<PACKED, 0, false>(p, rp);
 }
 
-// The packed instance on a RING-slot register ring (batches of up to kDeepRingTokens tokens).
-template <int RING, bool ROUTE = false>
+// The same on a RING-slot ring (batches of up to kDeepRingTokens tokens).
+template <bool PACKED, int RING, bool ROUTE>
 __global__ __launch_bounds__(kStreamWaves * 64) void gemm1_stream_dispatch_deep_kernel(GemmParams p, RouteParams rp) {
-  gemm1_stream_dispatch<true, RING, ROUTE>(p, rp);
+  gemm1_stream_dispatch<PACKED, RING, ROUTE>(p, rp);
 }
 
 // Requantises the fp32 SwiGLU rows: per row and COLS columns, scale = max(amax/448, 1e-12)
@@ -1121,23 +1128,26 @@ hipError_t launch_dispatch_instance(K kernel, std::atomic<int>& occ, const GemmP
 
 bool gemm1_dispatch_routes(int T) { return T <= kInlineRouteTokens; }
 
+// Batches of up to kDeepRingTokens tokens: the ring's depth and whether the kernel routes.
+template <bool PACKED>
+hipError_t launch_gemm1_deep(const GemmParams& p, const RouteParams& rp, bool route, hipStream_t s) {
+  static std::atomic<int> occ[4] = {};
+  static_assert(kDeeperRingTokens <= kInlineRouteTokens && kInlineRouteTokens <= kDeepRingTokens, "instances below");
+  if (p.T <= kDeeperRingTokens)
+    return route ? launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeeperRing, true>, occ[0], p, rp, s)
+                 : launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeeperRing, false>, occ[1], p, rp, s);
+  return route ? launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, true>, occ[2], p, rp, s)
+               : launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, false>, occ[3], p, rp, s);
+}
+
 hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, bool packed, bool route, hipStream_t s) {
-  static std::atomic<int> occ[8] = {};
+  static std::atomic<int> occ_packed{0}, occ_rows{0};
   if (p.T <= 0 || p.T > kFusedDispatchTokens || rp.rows_per_item != kFusedItemRows) return hipErrorInvalidValue;
   if (route && p.T > kInlineRouteTokens) return hipErrorInvalidValue;
-  const bool deeper = packed && p.T <= kDeeperRingTokens;
-  const bool deep = packed && !deeper && p.T <= kDeepRingTokens;
-  if (route) {
-    if (deeper) return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<kDeeperRing, true>, occ[0], p, rp, s);
-    if (deep) return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<kDeepRing, true>, occ[1], p, rp, s);
-    return launch_dispatch_instance(gemm1_stream_dispatch_kernel<false, true>, occ[2], p, rp, s);
-  }
-  if (deeper) return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<kDeeperRing>, occ[3], p, rp, s);
-  if (deep) return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<kDeepRing>, occ[4], p, rp, s);
-  if (packed) return launch_dispatch_instance(gemm1_stream_dispatch_kernel<true>, occ[5], p, rp, s);
-  return launch_dispatch_instance(gemm1_stream_dispatch_kernel<false>, occ[6], p, rp, s);
+  if (p.T <= kDeepRingTokens) return packed ? launch_gemm1_deep<true>(p, rp, route, s) : launch_gemm1_deep<false>(p, rp, route, s);
+  if (packed) return launch_dispatch_instance(gemm1_stream_dispatch_kernel<true>, occ_packed, p, rp, s);
+  return launch_dispatch_instance(gemm1_stream_dispatch_kernel<false>, occ_rows, p, rp, s);
 }
-static_assert(kInlineRouteTokens <= kDeepRingTokens, "routed batches of the packed copy take a deep ring");
 
 hipError_t launch_requant(const GemmParams& p, int rows_per_item, hipStream_t s) {
   if (rows_per_item > 32) return hipSuccess;   // the tile GEMM1 requantises in its epilogue

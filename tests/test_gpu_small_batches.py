@@ -1,0 +1,74 @@
+"""The smallest batches through moe_fp8_run and moe_fp8_run_packed, whose GEMM1 work-groups route the
+tokens themselves (up to 4) on rings of their own depth (6 slots up to 2 tokens, 4 up to 8): the
+top-k lists against the oracle, and lists, dispatch and output bit for bit against
+moe_fp8_run_profiled, which routes in a launch of its own."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import routing as orouting
+
+pytestmark = pytest.mark.gpu
+
+_STATE = {}
+
+
+def _weights():
+    import gpu_helpers as gh
+    if not _STATE:
+        w = gh.inputs.make_weights(911, torch.device("cuda:0"))
+        _STATE["w"], _STATE["p"] = w, gh.pkg.pack_weights(w[0], w[2])
+    return gh, _STATE["w"], _STATE["p"]
+
+
+def _call(gh, args, ws, packed, profiled):
+    lib = gh._lib.load()
+    p, n = (packed.data_ptr(), packed.numel()) if packed is not None else (None, 0)
+    if profiled:
+        events = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+        for e in events:
+            e.record()
+        rc = lib.moe_fp8_run_profiled(args, p, n, ws.ptr, ws.buffer.numel(), gh.stream(),
+                                      (ctypes.c_void_p * 4)(*[e.cuda_event for e in events]))
+    elif packed is not None:
+        rc = lib.moe_fp8_run_packed(args, p, n, ws.ptr, ws.buffer.numel(), gh.stream())
+    else:
+        rc = lib.moe_fp8_run(args, ws.ptr, ws.buffer.numel(), gh.stream())
+    gh._lib.check(rc, "run")
+
+
+@pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 8, 9])
+def test_small_batches(T, bias_dtype):
+    gh, w, packed = _weights()
+    dev = torch.device("cuda:0")
+    print(f"T={T} bias {bias_dtype}", flush=True)
+    for extreme in (False, True):
+        logits, bias, hq, hs = gh.inputs.make_activations(T, 60 + T, dev, 32, (1, 7))
+        if extreme:
+            # ties, saturated scores, and a last token with five finite candidates
+            logits = (logits * 4).round() * 30
+            logits[-1] = float("-inf")
+            logits[-1, 32:37] = torch.tensor([1.0, 2.0, 2.0, -1.0, 0.5], device=dev)
+        bias = bias.to(bias_dtype)
+        if extreme:
+            bias = bias.float().masked_fill(torch.arange(256, device=dev) >= 40, float("-inf")).to(bias_dtype)
+        want = None
+        for pk in (None, packed):
+            for profiled in (True, False):
+                out = torch.full((T, 7168), 7.0, dtype=torch.bfloat16, device=dev)
+                ws = gh.new_workspace(T, dev)
+                args = gh.make_args(logits, bias, hq, hs, w[0], w[1], w[2], w[3], 32, 2.5, out)
+                for _ in range(2):
+                    _call(gh, args, ws, pk, profiled)
+                torch.cuda.synchronize()
+                ids = gh.read(ws, "topk_ids", torch.int32, T * 8).reshape(T, 8)
+                tw = gh.read(ws, "topk_weights", torch.float32, T * 8).reshape(T, 8)
+                gh.check_dispatch(ws, ids, tw, 32, T)
+                got = (ids.tobytes(), tw.tobytes(), out.view(torch.int16).cpu().numpy().tobytes())
+                want = want or got
+                assert got == want, (T, extreme, pk is not None, profiled)
+        oid, ow = orouting.route(logits.cpu().numpy(), bias.float().cpu().numpy(), 2.5)
+        assert np.array_equal(ids, oid) and np.array_equal(tw.view(np.uint32), ow.view(np.uint32))
