@@ -234,8 +234,9 @@ int run_layer(const moe_fp8_args* args, void* workspace, size_t workspace_bytes,
     if (launch_route_dispatch(rp, stream) != hipSuccess || !mark(1)) return MOE_FP8_ELAUNCH;
     if (launch_gemm1(gp, L.rows_per_item, use_packed, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
   }
-  if (launch_requant(gp, L.rows_per_item, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
-  if (launch_gemm2(gp, L.rows_per_item, use_packed, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
+  const bool requant = !events && gemm2_requantises(args->num_tokens, use_packed);
+  if (!requant && launch_requant(gp, L.rows_per_item, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
+  if (launch_gemm2(gp, L.rows_per_item, use_packed, requant, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
   if (launch_combine(gp, L.rows_per_item, stream) != hipSuccess || !mark(3)) return MOE_FP8_ELAUNCH;
   return MOE_FP8_OK;
 }
@@ -321,7 +322,7 @@ int moe_fp8_gemm2_combine(const moe_fp8_args* args, void* workspace, size_t work
   if (args->num_tokens == 0) return MOE_FP8_OK;
   const GemmParams p = gemm_params(args, L, workspace);
   if (launch_requant(p, L.rows_per_item, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
-  if (launch_gemm2(p, L.rows_per_item, false, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
+  if (launch_gemm2(p, L.rows_per_item, false, false, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
   return launch_combine(p, L.rows_per_item, stream) == hipSuccess ? MOE_FP8_OK : MOE_FP8_ELAUNCH;
 }
 

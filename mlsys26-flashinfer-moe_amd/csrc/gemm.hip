@@ -64,7 +64,8 @@ constexpr int kStreamWaves = 4;                      // wavefronts per work-grou
 // and slower: T=64 110.3 against 105.5 us, T=16 55.6 against 54.3.
 // Requantising GEMM1's fp32 rows inside GEMM2 instead of in requant_kernel was measured
 // and is slower (T=64: GEMM2 + combine 68 -> 80 us): the per-element IEEE divisions, four
-// times the activation bytes and fewer resident wavefronts cost more than the launch.
+// times the activation bytes and fewer resident wavefronts cost more than the launch (batches
+// of one or two tokens, whose rows are few, do requantise there: gemm2_slice_kernel).
 // Columns per requantisation scale of the GEMM1 output on the streaming path: the
 // reference's 1x64 block (kernel.py:131-135); GEMM2 then applies two activation scales per
 // 128-wide K block.
@@ -518,7 +519,7 @@ struct FusedDispatch {
 // token per wavefront, instead of by a launch before it; work-group 0 also writes the lists. More
 // tokens than wavefronts would route one after another in all of them (1.9 us of a SIMD's issue
 // time per token). Layer on the packed copy, us: T=1 22.7 -> 21.2, T=2 38.5 -> 36.7, T=3 44.9 -> 43.8,
-// T=4 49.6 -> 48.1; the launch itself took 3.9 us, the routing here hides behind nothing.
+// T=4 49.6 -> 48.1.
 constexpr int kInlineRouteTokens = kStreamWaves;
 struct InlineRoute {
   float bias[kExpertsGlobal];
@@ -766,6 +767,7 @@ struct SliceStage {
   float sw[kSliceF];  // W2 block scale of the lane's four output rows of each fragment
   int tok;          // token of the lane's row
   float wt;         // routing weight of the lane's row
+  int r, ks;        // the lane's bucket row and the K-step (requantising instances: act comes from LDS)
 };
 
 // On the row-major weights the slice's 28 W2 rows of a K-step (rows past 28 repeating the
@@ -776,16 +778,60 @@ constexpr int kSliceLdsRows = 16 * kSliceF;                     // 32
 constexpr int kSliceLdsStep = kSliceLdsRows * 128;              // 4 KB per K-step
 constexpr int kSliceLdsDma = kSliceLdsRows / 8;                 // 4 DMA instructions
 
-template <bool RING>
+// TOKENS > 0 (batches of up to that many tokens): the kernel requantises GEMM1's rows itself, every
+// wavefront the 256 columns of its own K-steps of all rows (up to 8 per token, usually one or two)
+// into LDS, instead of reading what requant_kernel wrote; work-group 0 also writes them to the
+// workspace. This saves the launch (3.4 us and the gap before it), behind whose end the weight
+// stream could not start; it costs every CU the fp32 rows' bytes and ~0.25 us per row. Layer,
+// us, few local rows (random routing) and many (every token names 5 to 8 local experts):
+//                 packed, random   many         row-major, random   many
+//   T=1           21.2 -> 19.5     43.4 -> 42.4     35.7 -> 34.8   46.4 -> 46.4
+//   T=2           36.9 -> 35.6     53.2 -> 53.2     40.5 -> 40.1   55.7 -> 57.5
+//   T=3           43.8 -> 42.9     55.6 -> 56.8     46.1 -> 46.1
+//   T=4           48.5 -> 47.7     58.5 -> 60.9     50.6 -> 50.9   59.1 -> 64.0
+// so up to the sizes at which many rows lose nothing: 2 tokens packed, 1 row-major (whose LDS
+// ring the compiler drains around the rows' LDS stores).
+constexpr int kSlicePackedTokens = 2;
+constexpr int kSliceRowMajorTokens = 1;
+constexpr int kSliceActStride = kInter + 16;   // the 16 rows of a fragment load fall in distinct banks
+
+template <bool RING, int TOKENS>
 struct SliceShared {
-  float acc[kSliceParts][kFusedDispatchTokens][16 * kSliceF];
+  static constexpr int kTokens = TOKENS > 0 ? TOKENS : kFusedDispatchTokens;
+  static constexpr int kRows = TOKENS * kTopK;
+  static_assert(kRows % 2 == 0, "rows are requantised in groups of 2");
+  float acc[kSliceParts][kTokens][16 * kSliceF];
   uint8_t ring[RING ? kSliceParts : 0][kSliceRing * kSliceLdsStep];
+  uint8_t act[kRows][kSliceActStride];
+  float scale[kRows][kQuantBlocks];
 };
+static_assert(sizeof(SliceShared<true, kSliceRowMajorTokens>) <= 160 * 1024 &&
+              sizeof(SliceShared<false, kSlicePackedTokens>) <= 160 * 1024, "LDS of one CU");
+
+// kSliceRowGroup rows of GEMM1's output from row r0, 4 columns per thread (rows past the batch's
+// last slot repeat it; never used). Groups of 2, 4 of them in flight, against groups of 4, 2 in
+// flight: layer at T=1 19.9 -> 19.5 us, T=2 35.7 -> 35.6; one row at a time 19.6 / 36.3.
+constexpr int kSliceRowGroup = 2;
+constexpr int kSliceRowGroups = 4;
+
+__device__ __forceinline__ void load_swiglu_rows(const GemmParams& p, int r0, v4f (&x)[kSliceRowGroup]) {
+  const int last = p.T * kTopK - 1;
+#pragma unroll
+  for (int i = 0; i < kSliceRowGroup; ++i)
+    x[i] = *(reinterpret_cast<const v4f*>(p.swiglu + (size_t)min(r0 + i, last) * kInter) + threadIdx.x);
+}
 
 // PACKED: p.w2 is the packed copy of W2 (moe_fp8_run_packed).
-template <bool PACKED>
+template <bool PACKED, int TOKENS = 0>
 __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParams p) {
-  __shared__ __attribute__((aligned(1024))) SliceShared<!PACKED> sh;
+  static_assert(kSliceParts * 64 * 4 == kInter, "a row is 4 columns per thread");
+  __shared__ __attribute__((aligned(1024))) SliceShared<!PACKED, TOKENS> sh;
+  // loaded before their number is known
+  v4f rows_in[kSliceRowGroups][kSliceRowGroup];
+  if constexpr (TOKENS > 0) {
+#pragma unroll
+    for (int h = 0; h < kSliceRowGroups; ++h) load_swiglu_rows(p, h * kSliceRowGroup, rows_in[h]);
+  }
   auto& acc_lds = sh.acc;
   const int lane = threadIdx.x & 63;
   const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -795,6 +841,46 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
   const int4 my_item = lane < n_items ? reinterpret_cast<const int4*>(p.work_items)[lane] : make_int4(0, 0, 0, 0);
   const int nsteps = n_items * kSliceSteps;
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
+  // requant_kernel's operations on 4 columns per thread, 16 lanes per block. A wavefront's threads
+  // hold exactly the 256 columns of its own K-steps, so nothing is shared between wavefronts.
+  static_assert(kSliceSteps * 128 == 64 * 4 && kQuantCols == 16 * 4, "columns of a wavefront");
+  auto requantise = [&]() __attribute__((always_inline)) {
+    const int tid = threadIdx.x;
+    const int n_rows = min(p.counters[kCtrAssign], sh.kRows);
+    for (int r0 = 0; r0 < n_rows; r0 += kSliceRowGroups * kSliceRowGroup) {
+#pragma unroll
+      for (int h = 0; h < kSliceRowGroups; ++h) {
+        const int rg = r0 + h * kSliceRowGroup;
+        if (rg >= n_rows) break;
+        v4f(&x)[kSliceRowGroup] = rows_in[h];
+        uint32_t w[kSliceRowGroup];
+        float scale[kSliceRowGroup];
+#pragma unroll
+        for (int i = 0; i < kSliceRowGroup; ++i) {
+          const v4f c = x[i];
+          float amax = fmaxf(fmaxf(fabsf(c[0]), fabsf(c[1])), fmaxf(fabsf(c[2]), fabsf(c[3])));
+          amax = fmaxf(amax, dpp_f32<kDppXor1>(amax));
+          amax = fmaxf(amax, dpp_f32<kDppXor2>(amax));
+          amax = fmaxf(amax, dpp_f32<kDppHalfMirror>(amax));
+          amax = fmaxf(amax, dpp_f32<kDppMirror>(amax));
+          scale[i] = fmaxf(amax / 448.0f, 1e-12f);
+          w[i] = pack_fp8x4(c[0] / scale[i], c[1] / scale[i], c[2] / scale[i], c[3] / scale[i]);
+        }
+        if (rg + kSliceRowGroups * kSliceRowGroup < n_rows) load_swiglu_rows(p, rg + kSliceRowGroups * kSliceRowGroup, x);
+        const bool head = tid % (kQuantCols / 4) == 0;
+#pragma unroll
+        for (int i = 0; i < kSliceRowGroup; ++i) {   // rows past the last are written to LDS, never read
+          const int r = rg + i;
+          *reinterpret_cast<uint32_t*>(&sh.act[r][4 * tid]) = w[i];
+          if (head) sh.scale[r][tid / (kQuantCols / 4)] = scale[i];
+          if (blockIdx.x == 0 && r < n_rows) {
+            reinterpret_cast<uint32_t*>(p.act + (size_t)r * kInter)[tid] = w[i];
+            if (head) p.act_scale[(size_t)r * kQuantBlocks + tid / (kQuantCols / 4)] = scale[i];
+          }
+        }
+      }
+    }
+  };
   for (int slice = blockIdx.x; slice < kHiddenSlices; slice += gridDim.x) {
     const int h0 = slice * kSliceRows;
     float* my_acc = &acc_lds[q][0][0];
@@ -821,7 +907,9 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
           const int orow = h0 + min(16 * f + 4 * (lane >> 4), kSliceRows - 1);   // first output row
           g.sw[f] = p.w2_scale[((size_t)e * kHBlocks + orow / kBlock) * kIBlocks + ks];
         }
-        g.sa = *reinterpret_cast<const float2*>(p.act_scale + (size_t)r * kQuantBlocks + 2 * ks);
+        if constexpr (TOKENS == 0) g.sa = *reinterpret_cast<const float2*>(p.act_scale + (size_t)r * kQuantBlocks + 2 * ks);
+        g.r = r;
+        g.ks = ks;
         g.tok = p.sorted_token[r];
         g.wt = p.sorted_weight[r];
         if constexpr (!PACKED) {
@@ -844,11 +932,15 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
                                       ((hr & 15) + 16 * (lane >> 4)) * 32);
           }
         }
-        g.a = load_frag(p.act + (size_t)r * kInter + ks * 128 + (lane >> 4) * 16);
+        if constexpr (TOKENS == 0) g.a = load_frag(p.act + (size_t)r * kInter + ks * 128 + (lane >> 4) * 16);
       };
       SliceStage ring[kSliceRing];
 #pragma unroll
       for (int u = 0; u < kSliceRing - 1; ++u) issue(u, ring[u]);
+      if constexpr (TOKENS > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (slice == (int)blockIdx.x) requantise();
+      }
       v4f acc[kSliceF];
 #pragma unroll
       for (int f = 0; f < kSliceF; ++f) acc[f] = zero;
@@ -872,8 +964,10 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
             // in flight. Covering every load of step st0 + u here also keeps the compiler
             // from waiting on the rest itself, which it would do with vmcnt(0) while the
             // ring's DMAs are in flight.
-            if (u == kSliceSteps - 2) wait_vm<kSliceLdsDma + 7>();
-            else wait_vm<kSliceLdsDma + 5>();
+            // (requantising instances load no act and no act scales: 3 fewer)
+            constexpr int kAct = TOKENS > 0 ? 0 : 3;
+            if (u == kSliceSteps - 2) wait_vm<kSliceLdsDma + 4 + kAct>();
+            else wait_vm<kSliceLdsDma + 2 + kAct>();
             __builtin_amdgcn_sched_barrier(0);
             const uint8_t* b = sh.ring[q] + (u % kSliceRing) * kSliceLdsStep;
 #pragma unroll
@@ -884,12 +978,18 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
           // the act fragment's two 64-column halves carry their own scales: one MFMA per
           // half, the other half's bytes zeroed (lanes hold bytes [16j, 16j+16) of the first
           // half in a[0..3] and of the second in a[4..7])
+          v8i a = g.a;
+          float2 sa = g.sa;
+          if constexpr (TOKENS > 0) {
+            a = load_frag(&sh.act[g.r][g.ks * 128 + (lane >> 4) * 16]);
+            sa = *reinterpret_cast<const float2*>(&sh.scale[g.r][2 * g.ks]);
+          }
           const v4i kZero4 = {0, 0, 0, 0};
-          const v8i a_lo = join(lo_half(g.a), kZero4);
-          const v8i a_hi = join(kZero4, hi_half(g.a));
+          const v8i a_lo = join(lo_half(a), kZero4);
+          const v8i a_hi = join(kZero4, hi_half(a));
 #pragma unroll
           for (int f = 0; f < kSliceF; ++f) {
-            const float sc_lo = g.sa.x * g.sw[f], sc_hi = g.sa.y * g.sw[f];
+            const float sc_lo = sa.x * g.sw[f], sc_hi = sa.y * g.sw[f];
             const v4f d_lo = mfma16x16x128_fp8(wf[f], a_lo, zero);
             const v4f d_hi = mfma16x16x128_fp8(wf[f], a_hi, zero);
             acc[f] += d_lo * sc_lo;
@@ -1149,6 +1249,9 @@ hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, boo
   return launch_dispatch_instance(gemm1_stream_dispatch_kernel<false>, occ_rows, p, rp, s);
 }
 
+bool gemm2_requantises(int T, bool packed) { return T <= (packed ? kSlicePackedTokens : kSliceRowMajorTokens); }
+static_assert(kSlicePackedTokens <= kFusedDispatchTokens && kSliceRowMajorTokens <= kFusedDispatchTokens, "slice batches");
+
 hipError_t launch_requant(const GemmParams& p, int rows_per_item, hipStream_t s) {
   if (rows_per_item > 32) return hipSuccess;   // the tile GEMM1 requantises in its epilogue
   int grid = p.T * kTopK;                      // rows of the SwiGLU buffer
@@ -1160,13 +1263,16 @@ hipError_t launch_requant(const GemmParams& p, int rows_per_item, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_gemm2(const GemmParams& p, int rows_per_item, bool packed, hipStream_t s) {
+hipError_t launch_gemm2(const GemmParams& p, int rows_per_item, bool packed, bool requant, hipStream_t s) {
+  if (requant && rows_per_item != kFusedItemRows) return hipErrorInvalidValue;
   if (rows_per_item > 32) return launch_gemm2_tile(p, rows_per_item, s);
   if (rows_per_item == kFusedItemRows) {
     // up to 64 tokens: GEMM2 with the combine, one work-group per 32-row hidden slice
     if (p.T > kFusedDispatchTokens) return hipErrorInvalidValue;
-    if (packed) hipLaunchKernelGGL(gemm2_slice_kernel<true>, dim3(kHiddenSlices), dim3(kSliceParts * 64), 0, s, p);
-    else hipLaunchKernelGGL(gemm2_slice_kernel<false>, dim3(kHiddenSlices), dim3(kSliceParts * 64), 0, s, p);
+    if (requant && !gemm2_requantises(p.T, packed)) return hipErrorInvalidValue;
+    const auto kernel = packed ? (requant ? gemm2_slice_kernel<true, kSlicePackedTokens> : gemm2_slice_kernel<true>)
+                               : (requant ? gemm2_slice_kernel<false, kSliceRowMajorTokens> : gemm2_slice_kernel<false>);
+    hipLaunchKernelGGL(kernel, dim3(kHiddenSlices), dim3(kSliceParts * 64), 0, s, p);
     return hipGetLastError();
   }
   return launch_stream<kG2>(p, rows_per_item, packed, s);

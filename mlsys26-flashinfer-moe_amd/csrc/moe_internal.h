@@ -4,9 +4,10 @@
 //   caller tensors   : the contract of kernel.py:591-607 (see include/moe_fp8.h)
 //   workspace arrays : moe_fp8_layout offsets; every array is 256-byte aligned.
 // Kernels of one call run in this order on one stream:
-//   T <= 64 (moe_fp8_run): route_wide_kernel -> gemm1_stream_dispatch_kernel (GEMM1 that
-//   rebuilds the dispatch itself) -> requant_kernel -> gemm2_slice_kernel (GEMM2 and the
-//   combine); otherwise
+//   T <= 64 (moe_fp8_run): [route_wide_kernel] -> gemm1_stream_dispatch_kernel (GEMM1 that
+//   rebuilds the dispatch itself; up to 4 tokens it routes them too) -> [requant_kernel] ->
+//   gemm2_slice_kernel (GEMM2 and the combine; up to 2 tokens, or 1 on row-major weights, it
+//   requantises too); otherwise
 //   route_wide_kernel -> dispatch_small_kernel (T <= 256) | route_kernel -> place_kernel
 //   -> GEMM1 -> [requant_kernel] -> GEMM2 -> [combine_kernel]
 // where, with <= 32 rows per work item, GEMM1 is gemm_stream_kernel<1> and leaves fp32 SwiGLU
@@ -156,7 +157,10 @@ hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, boo
 bool gemm1_dispatch_routes(int T);
 hipError_t launch_requant(const GemmParams& p, int rows_per_item, hipStream_t s);
 // packed (items of up to 32 rows): p.w2 is the packed copy of W2.
-hipError_t launch_gemm2(const GemmParams& p, int rows_per_item, bool packed, hipStream_t s);
+// requant: the kernel requantises GEMM1's rows too (where gemm2_requantises(T, packed)), without
+// launch_requant before it.
+hipError_t launch_gemm2(const GemmParams& p, int rows_per_item, bool packed, bool requant, hipStream_t s);
+bool gemm2_requantises(int T, bool packed);
 // The packed copy of W13 and W2 read by the decode kernels (moe_fp8_pack_weights).
 size_t packed_weights_bytes();
 hipError_t launch_pack_weights(const uint8_t* w13, const uint8_t* w2, uint8_t* packed, hipStream_t s);

@@ -1,7 +1,9 @@
 """The smallest batches through moe_fp8_run and moe_fp8_run_packed, whose GEMM1 work-groups route the
-tokens themselves (up to 4) on rings of their own depth (6 slots up to 2 tokens, 4 up to 8): the
-top-k lists against the oracle, and lists, dispatch and output bit for bit against
-moe_fp8_run_profiled, which routes in a launch of its own."""
+tokens themselves (up to 4) on rings of their own depth (6 slots up to 2 tokens, 4 up to 8), and whose
+GEMM2 work-groups requantise GEMM1's rows (1 token, packed 2): the top-k lists against the oracle,
+lists, dispatch and output bit for bit against moe_fp8_run_profiled, which routes in a launch of its
+own, and the requantised rows bit for bit against the formula and the output against the same
+tokens in a larger batch, which requant_kernel requantises."""
 import ctypes
 
 import numpy as np
@@ -72,3 +74,32 @@ def test_small_batches(T, bias_dtype):
                 assert got == want, (T, extreme, pk is not None, profiled)
         oid, ow = orouting.route(logits.cpu().numpy(), bias.float().cpu().numpy(), 2.5)
         assert np.array_equal(ids, oid) and np.array_equal(tw.view(np.uint32), ow.view(np.uint32))
+
+
+@pytest.mark.parametrize("boosted", [(), (1, 7), (1, 4, 7, 9, 12, 15, 20, 22)])
+@pytest.mark.parametrize("T", [1, 2, 3])
+def test_requantised_rows(T, boosted):
+    gh, w, packed = _weights()
+    dev = torch.device("cuda:0")
+    big = 9
+    logits, bias, hq, hs = gh.inputs.make_activations(big, 80, dev, 32, boosted)
+    for pk in (None, packed):
+        outs = []
+        for n in (T, big):
+            print(f"T={n} packed {pk is not None}", flush=True)
+            out = torch.full((n, 7168), 7.0, dtype=torch.float32, device=dev)
+            ws = gh.new_workspace(n, dev)
+            args = gh.make_args(logits[:n].contiguous(), bias, hq[:n].contiguous(), hs[:, :n].contiguous(),
+                                w[0], w[1], w[2], w[3], 32, 2.5, out)
+            for _ in range(2):
+                _call(gh, args, ws, pk, False)
+            torch.cuda.synchronize()
+            outs.append(out)
+            rows = int(gh.read(ws, "counters", torch.int32, 2)[1])
+            x = torch.from_numpy(gh.read(ws, "swiglu", torch.float32, rows * 2048).copy()).reshape(rows, 32, 64)
+            scale = (x.abs().amax(-1) / 448.0).clamp_min(1e-12)
+            q = (x / scale[..., None]).to(torch.float8_e4m3fn).view(torch.uint8).reshape(rows, 2048)
+            assert rows > 0 or not boosted
+            assert np.array_equal(gh.read(ws, "act", torch.uint8, rows * 2048).reshape(rows, 2048), q.numpy())
+            assert np.array_equal(gh.read(ws, "act_scale", torch.float32, rows * 32).reshape(rows, 32), scale.numpy())
+        assert torch.equal(outs[0], outs[1][:T])
