@@ -8,7 +8,8 @@
 //   rebuilds the dispatch itself; up to 4 tokens it routes them too) -> [requant_kernel] ->
 //   gemm2_slice_kernel (GEMM2 and the combine; up to 2 tokens, or 1 on row-major weights, it
 //   requantises too); otherwise
-//   route_wide_kernel -> dispatch_small_kernel (T <= 256) | route_kernel -> place_kernel
+//   route_wide_kernel -> dispatch_small_kernel (T <= 128) | route_parts_kernel (T <= 2048) or
+//   route_kernel -> place_kernel
 //   -> GEMM1 -> [requant_kernel] -> GEMM2 -> [combine_kernel]
 // where, with <= 32 rows per work item, GEMM1 is gemm_stream_kernel<1> and leaves fp32 SwiGLU
 // rows for requant_kernel, and GEMM2 is gemm2_slice_kernel (16-row items, up to 64 tokens)
@@ -35,14 +36,16 @@ constexpr int kBlock = MOE_FP8_BLOCK;          // 128
 constexpr int kHBlocks = MOE_FP8_H_BLOCKS;     // 56
 constexpr int kIBlocks = MOE_FP8_I_BLOCKS;     // 16
 
-// Routing: up to kWideRouteTokens tokens one token per wavefront (4 per work-group), above
+// Routing: up to kWideDispatchTokens tokens one token per wavefront (4 per work-group), above
 // that 16 lanes per token and 16 tokens per work-group of 4 wavefronts; the one-work-group
 // dispatch of small batches uses 1024 threads.
-constexpr int kWideRouteTokens = 256;
 constexpr int kRouteTokensPerBlock = 16;
 constexpr int kRouteThreads = 1024;
-// Up to this many tokens routing and dispatch run in a single work-group (one launch).
-constexpr int kSinglePassTokens = 256;
+constexpr int kWideDispatchTokens = 2048;
+// Up to this many tokens the dispatch runs in a single work-group, one slot per thread; with
+// several per thread it is the slower one (layer, us, against place_kernel: T=100 158.6 / 158.8,
+// 128 169.8 / 170.0, 200 189.8 / 186.8, 256 203.1 / 199.9).
+constexpr int kSinglePassTokens = 128;
 // Up to this many tokens moe_fp8_run launches routing alone, and every GEMM1 work-group
 // rebuilds the dispatch in LDS (work-group 0 also writes it to the workspace).
 constexpr int kFusedDispatchTokens = 64;

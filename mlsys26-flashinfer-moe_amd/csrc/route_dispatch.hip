@@ -1,18 +1,17 @@
 // Routing and dispatch for the fused MoE layer (gfx950).
 //
 // The DeepSeek-V3 no-aux grouped routing (kernel.py:428-542) runs with branch-free DPP
-// reductions: up to 256 tokens one token per wavefront (route_wide_kernel: 4 experts per lane,
-// the shortest dependent chain per token), above that sixteen lanes per token and four
-// tokens per wavefront (route_kernel, which also records per-work-group histograms and ranks
-// for the multi-work-group dispatch). Dispatch then histograms the local assignments, scans
-// them into CSR offsets, builds the GEMM work list and places every assignment in its bucket:
-//   T <= 256 (or given top-k lists): route_wide_kernel -> dispatch_small_kernel, which does the
-//             whole dispatch in one work-group, in LDS (up to 64 tokens moe_fp8_run rebuilds the
-//             dispatch inside GEMM1 instead);
-//   larger T: route_kernel (also per work-group histograms and ranks) -> place_kernel (above
-//             16384 tokens with block_scan_kernel between them, which keeps the cost linear in T)
-//             (each work-group reduces the histograms it needs). No kernel synchronises
-//             across work-groups.
+// reductions: up to 2048 tokens one token per wavefront (route_wide: 4 experts per lane, the
+// shortest dependent chain per token), above that sixteen lanes per token and four tokens per
+// wavefront. Dispatch then histograms the local assignments, scans them into CSR offsets,
+// builds the GEMM work list and places every assignment in its bucket:
+//   T <= 128: route_wide_kernel -> dispatch_small_kernel, which does the whole dispatch in one
+//             work-group (up to 64 tokens moe_fp8_run rebuilds the dispatch inside GEMM1 instead);
+//   larger T: route_parts_kernel up to 2048 tokens, route_kernel above (both also record
+//             per-work-group histograms and ranks) -> place_kernel (above 16384 tokens with
+//             block_scan_kernel between them, which keeps the cost linear in T) (each
+//             work-group reduces the histograms it needs). No kernel synchronises across
+//             work-groups.
 //
 // The order inside an expert's bucket is ascending token (then slot), i.e. a stable sort
 // by expert of the flat top-k list; the reference's atomic scatter (kernel.py:288-324)
@@ -282,28 +281,64 @@ __global__ __launch_bounds__(kRouteWaves * 64) void route_kernel(RouteParams p) 
   }
 }
 
-// Dispatch of up to kRouteThreads slots held one per thread (slot tid = token tid/8, top-k
-// position tid%8; le < 0: not a local expert): local counts, stable ranks, CSR offsets, the
-// work list and the placement. The whole work-group calls this.
-__device__ __forceinline__ void dispatch_slots(const RouteParams& p, int le, float w, int nslots,
-                                               int (*s_wcnt)[kExpertsLocal], int* s_cnt, int* s_start) {
+// The same for batches of kSinglePassTokens to kWideDispatchTokens tokens, one token per wavefront (route_wide) and
+// kWideTokens per work-group, a quarter of a 16-token block: the ranks are those among the
+// work-group's 32 slots, and its counts (at most 32) are byte q of the block's 32 histogram
+// entries, which place_kernel<.., true> sums with v_sad_u8. Four work-groups per block, also past the
+// last token, so that every byte is written. What bounds it is the dependent chain of a token's
+// eight argmax rounds, on a chip that is mostly idle: four tokens per wavefront and 16 per
+// work-group make that chain longer and fill 57 CUs at 901 tokens, these 226. Layer, us,
+// against route_kernel: T=300 204.3 -> 202.1, 901 242.0 -> 240.2, 1500 268.0 -> 266.3, 2048 301.2 ->
+// 299.4; 3000 351.3 -> 352.0, 4000 397.6 -> 399.1 (2.5 times the instructions per token).
+constexpr int kWideTokens = 4;
+constexpr int kWideParts = kRouteTokensPerBlock / kWideTokens;   // 4 bytes of an entry
+static_assert(kWideParts == 4 && kWideTokens * kTopK <= 64, "one byte per part, one wavefront's slots");
+
+__global__ __launch_bounds__(kWideTokens * 64) void route_parts_kernel(RouteParams p) {
+  __shared__ __attribute__((aligned(16))) float s_bias[kExpertsGlobal];
+  __shared__ int s_le[kWideTokens * kTopK];
   const int tid = threadIdx.x;
-  // the 8 slots of token tid/8 are 8 consecutive lanes, so one ballot gives every token's
-  // local count
-  const uint64_t m = __ballot(le >= 0);
-  if ((tid & 7) == 0 && tid < nslots) p.token_nlocal[tid >> 3] = __popcll((m >> (lane_id() & 56)) & 0xFFull);
-  const int r = block_rank(le, kRouteThreads / 64, s_wcnt, s_cnt);
-  if (tid < kExpertsLocal) finish_counts(p, tid, s_cnt[tid], s_start);
-  __syncthreads();
-  if (le >= 0) {
-    const int pos = s_start[le] + r;
-    p.sorted_token[pos] = tid >> 3;
-    p.sorted_weight[pos] = w;
-    p.sorted_slot[pos] = tid;
+  const int lane = lane_id();
+  const int wave = tid >> 6;
+  const int tw = blockIdx.x * kWideTokens + wave;
+  const int t = min(tw, p.T - 1);   // wavefronts past the end recompute the last token
+  const bool slot_lane = tw < p.T && lane < kTopK;
+  float4 lg = {0.f, 0.f, 0.f, 0.f};
+  if (!p.skip_routing) lg = reinterpret_cast<const float4*>(p.logits + (size_t)t * kExpertsGlobal)[lane];
+  stage_bias(p, s_bias);
+  int id = -1;
+  if (!p.skip_routing) {
+    float w = 0.f;
+    id = route_wide(p, s_bias, t, lg, w);
+    if (slot_lane) {
+      p.topk_ids[t * kTopK + lane] = id;
+      p.topk_w[t * kTopK + lane] = w;
+    }
+  } else if (slot_lane) {
+    id = p.topk_ids[t * kTopK + lane];
   }
+  const int le = slot_lane ? local_of(id, p.offset) : -1;
+  const uint64_t m = __ballot(le >= 0);
+  if (lane == 0 && tw < p.T) p.token_nlocal[tw] = __popcll(m);
+  if (lane < kTopK) s_le[wave * kTopK + lane] = le;
+  __syncthreads();
+  if (wave != 0) return;
+  const int my_le = lane < kWideTokens * kTopK ? s_le[lane] : -1;
+  const uint64_t lt = lanemask_lt();
+  int rank = 0, cnt = 0;
+#pragma unroll 4
+  for (int e = 0; e < kExpertsLocal; ++e) {
+    const uint64_t me = __ballot(my_le == e);
+    if (my_le == e) rank = __popcll(me & lt);
+    if (lane == e) cnt = __popcll(me);
+  }
+  if (my_le >= 0) p.slot_rank[blockIdx.x * kWideTokens * kTopK + lane] = rank;
+  if (lane < kExpertsLocal)
+    reinterpret_cast<uint8_t*>(p.block_count)[((blockIdx.x / kWideParts) * kExpertsLocal + lane) * 4 +
+                                              blockIdx.x % kWideParts] = (uint8_t)cnt;
 }
 
-// Routing of up to kWideRouteTokens tokens, one token per wavefront and four per work-group
+// Routing of up to kSinglePassTokens tokens, one token per wavefront and four per work-group
 // (route_wide): top-k lists only, the dispatch follows in its own kernel or in GEMM1.
 __global__ __launch_bounds__(256) void route_wide_kernel(RouteParams p) {
   __shared__ __attribute__((aligned(16))) float s_bias[kExpertsGlobal];
@@ -320,57 +355,32 @@ __global__ __launch_bounds__(256) void route_wide_kernel(RouteParams p) {
   }
 }
 
-// Dispatch of small batches (T <= kSinglePassTokens) in one work-group, from the top-k
-// lists in the workspace: local counts, stable ranks (1024 slots at a time), CSR offsets,
-// the work list and the placement, without leaving the work-group.
+// Dispatch of small batches (T <= kSinglePassTokens) in one work-group, from the top-k lists in the
+// workspace, one slot per thread (slot tid = token tid/8, top-k position tid%8): local counts, stable
+// ranks, CSR offsets, the work list and the placement.
+static_assert(kSinglePassTokens * kTopK <= kRouteThreads, "one slot per thread");
+
 __global__ __launch_bounds__(kRouteThreads) void dispatch_small_kernel(RouteParams p) {
-  __shared__ int s_le[kSinglePassTokens * kTopK];
-  __shared__ int s_rank[kSinglePassTokens * kTopK];
-  __shared__ float s_w[kSinglePassTokens * kTopK];
   __shared__ int s_wcnt[16][kExpertsLocal];
   __shared__ int s_cnt[kExpertsLocal];
-  __shared__ int s_base[kExpertsLocal];
   __shared__ int s_start[kExpertsLocal + 1];
 
   const int tid = threadIdx.x;
   const int nslots = p.T * kTopK;
-  if (nslots <= kRouteThreads) {
-    // one slot per thread, kept in registers
-    const int le = tid < nslots ? local_of(p.topk_ids[tid], p.offset) : -1;
-    const float w = tid < nslots ? p.topk_w[tid] : 0.f;
-    dispatch_slots(p, le, w, nslots, s_wcnt, s_cnt, s_start);
-    return;
-  }
-  for (int slot = tid; slot < nslots; slot += kRouteThreads) {
-    s_le[slot] = local_of(p.topk_ids[slot], p.offset);
-    s_w[slot] = p.topk_w[slot];
-  }
-  if (tid < kExpertsLocal) s_base[tid] = 0;
+  const int le = tid < nslots ? local_of(p.topk_ids[tid], p.offset) : -1;
+  const float w = tid < nslots ? p.topk_w[tid] : 0.f;
+  // the 8 slots of token tid/8 are 8 consecutive lanes, so one ballot gives every token's
+  // local count
+  const uint64_t m = __ballot(le >= 0);
+  if ((tid & 7) == 0 && tid < nslots) p.token_nlocal[tid >> 3] = __popcll((m >> (lane_id() & 56)) & 0xFFull);
+  const int r = block_rank(le, kRouteThreads / 64, s_wcnt, s_cnt);
+  if (tid < kExpertsLocal) finish_counts(p, tid, s_cnt[tid], s_start);
   __syncthreads();
-  for (int t = tid; t < p.T; t += kRouteThreads) {
-    int n = 0;
-#pragma unroll
-    for (int k = 0; k < kTopK; ++k) n += s_le[t * kTopK + k] >= 0 ? 1 : 0;
-    p.token_nlocal[t] = n;
-  }
-  for (int c0 = 0; c0 < nslots; c0 += kRouteThreads) {
-    const int slot = c0 + tid;
-    const int le = slot < nslots ? s_le[slot] : -1;
-    const int r = block_rank(le, kRouteThreads / 64, s_wcnt, s_cnt);
-    if (le >= 0) s_rank[slot] = s_base[le] + r;
-    __syncthreads();
-    if (tid < kExpertsLocal) s_base[tid] += s_cnt[tid];
-    __syncthreads();
-  }
-  if (tid < kExpertsLocal) finish_counts(p, tid, s_base[tid], s_start);
-  __syncthreads();
-  for (int slot = tid; slot < nslots; slot += kRouteThreads) {
-    const int le = s_le[slot];
-    if (le < 0) continue;
-    const int pos = s_start[le] + s_rank[slot];
-    p.sorted_token[pos] = slot / kTopK;
-    p.sorted_weight[pos] = s_w[slot];
-    p.sorted_slot[pos] = slot;
+  if (le >= 0) {
+    const int pos = s_start[le] + r;
+    p.sorted_token[pos] = tid >> 3;
+    p.sorted_weight[pos] = w;
+    p.sorted_slot[pos] = tid;
   }
 }
 
@@ -389,8 +399,11 @@ static_assert(kRouteTokensPerBlock * kTopK <= kPlaceThreads, "one slot per threa
 // already turned block_count into per-work-group exclusive prefixes and written the CSR
 // offsets, so that each work-group reads its 32 prefixes instead of reducing every
 // histogram (which costs O(work-groups^2) in all).
-template <bool SCANNED>
+// PARTS (route_parts_kernel): a histogram entry is four counts in bytes, of the block's quarters.
+template <bool SCANNED, bool PARTS = false>
 __global__ __launch_bounds__(kPlaceThreads) void place_kernel(RouteParams p) {
+  static_assert(!(SCANNED && PARTS), "block_scan_kernel sums whole entries");
+  __shared__ uint32_t s_own[kExpertsLocal];
   __shared__ int s_pre[kPlaceGroups][kExpertsLocal];
   __shared__ int s_tot[kPlaceGroups][kExpertsLocal];
   __shared__ int s_prefix[kExpertsLocal];
@@ -433,8 +446,15 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(RouteParams p) {
     }
 #pragma unroll
     for (int i = 0; i < kScanBatch; ++i) {
-      tot += v[i];
-      pre += (b0 + i * kPlaceGroups < b) ? v[i] : 0;
+      const int bb = b0 + i * kPlaceGroups;
+      if constexpr (PARTS) {
+        tot = __builtin_amdgcn_sad_u8(v[i], 0, tot);
+        pre = __builtin_amdgcn_sad_u8(bb < b ? v[i] : 0, 0, pre);
+        if (bb == b) s_own[e] = v[i];
+      } else {
+        tot += v[i];
+        pre += bb < b ? v[i] : 0;
+      }
     }
   }
   s_pre[j][e] = pre;
@@ -463,7 +483,9 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(RouteParams p) {
   }
   __syncthreads();
   if (le < 0) return;
-  const int pos = s_start[le] + s_prefix[le] + rank;
+  int pos = s_start[le] + s_prefix[le] + rank;
+  // the slots of the block's earlier quarters
+  if constexpr (PARTS) pos += __builtin_amdgcn_sad_u8(s_own[le] & ((1u << (8 * (tid / (kWideTokens * kTopK)))) - 1), 0, 0);
   p.sorted_token[pos] = tok;
   p.sorted_weight[pos] = w;
   p.sorted_slot[pos] = s;
@@ -519,11 +541,10 @@ __global__ __launch_bounds__(kBlockScanThreads) void block_scan_kernel(RoutePara
   if (tid < kExpertsLocal) finish_counts(p, tid, tot, s_start);
 }
 
-// top-k lists only (no dispatch), for batches of up to kWideRouteTokens tokens
-static_assert(kWideRouteTokens >= kSinglePassTokens && kWideRouteTokens >= kFusedDispatchTokens,
-              "every batch routed without ranks fits route_wide_kernel");
+// top-k lists only (no dispatch), for batches of up to kSinglePassTokens tokens
+static_assert(kSinglePassTokens >= kFusedDispatchTokens, "every batch routed without ranks fits route_wide_kernel");
 static hipError_t launch_route_lists(const RouteParams& p, hipStream_t s) {
-  if (p.T > kWideRouteTokens) return hipErrorInvalidValue;
+  if (p.T > kSinglePassTokens) return hipErrorInvalidValue;
   hipLaunchKernelGGL(route_wide_kernel, dim3((p.T + 3) / 4), dim3(256), 0, s, p);
   return hipGetLastError();
 }
@@ -534,13 +555,16 @@ hipError_t launch_route_dispatch(const RouteParams& p, hipStream_t s) {
   if (p.single_pass) {
     if (!p.skip_routing && launch_route_lists(p, s) != hipSuccess) return hipGetLastError();
     hipLaunchKernelGGL(dispatch_small_kernel, dim3(1), dim3(kRouteThreads), 0, s, p);
+  } else if (p.T <= kWideDispatchTokens) {
+    hipLaunchKernelGGL(route_parts_kernel, dim3(p.nblocks * kWideParts), dim3(kWideTokens * 64), 0, s, p);
+    hipLaunchKernelGGL((place_kernel<false, true>), dim3(p.nblocks), dim3(kPlaceThreads), 0, s, p);
   } else {
     hipLaunchKernelGGL(route_kernel, dim3(p.nblocks), dim3(kRouteWaves * 64), 0, s, p);
     if (p.nblocks > kPlaceDirectBlocks) {
       hipLaunchKernelGGL(block_scan_kernel, dim3(1), dim3(kBlockScanThreads), 0, s, p);
-      hipLaunchKernelGGL(place_kernel<true>, dim3(p.nblocks), dim3(kPlaceThreads), 0, s, p);
+      hipLaunchKernelGGL((place_kernel<true>), dim3(p.nblocks), dim3(kPlaceThreads), 0, s, p);
     } else {
-      hipLaunchKernelGGL(place_kernel<false>, dim3(p.nblocks), dim3(kPlaceThreads), 0, s, p);
+      hipLaunchKernelGGL((place_kernel<false>), dim3(p.nblocks), dim3(kPlaceThreads), 0, s, p);
     }
   }
   return hipGetLastError();
