@@ -72,6 +72,39 @@ __device__ __forceinline__ uint64_t dpp_u64_rows(uint64_t v) {
   return ((uint64_t)hi << 32) | lo;
 }
 
+// Inclusive sum over lanes 0..31 (which must all be active), by DPP row shifts and one row broadcast:
+// a shuffle through the data-share unit costs several times a step's latency.
+__device__ __forceinline__ int scan32(int v) {
+  v += dpp_i32<0x111>(v);   // row_shr:1
+  v += dpp_i32<0x112>(v);
+  v += dpp_i32<0x114>(v);
+  v += dpp_i32<0x118>(v);
+  v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xA, 0xF, false);
+  return v;
+}
+
+// Stable rank of each lane's slot among the wavefront's slots of the same local expert (le < 0: not
+// local), and the wavefront's 32 counts in `cnt` (LDS): one ballot per distinct local expert of the
+// wavefront, a few of the 32 as a rule. Against a ballot for each of the 32 (with the scans by
+// shuffle): layer at T=80 162.0 -> 160.8 us, 128 168.7 -> 167.4, 901 239.4 -> 238.8, 8192 583.8 -> 582.2,
+// skewed T=128 220.0 -> 218.7. GEMM1's own dispatch keeps its shuffles: with scan32 T=16 68.7 -> 68.5,
+// but skewed T=64 170.4 -> 170.8.
+__device__ __forceinline__ int wave_rank(int le, int* cnt) {
+  const int lane = lane_id();
+  const uint64_t lt = lanemask_lt();
+  if (lane < kExpertsLocal) cnt[lane] = 0;
+  int rank = 0;
+  uint64_t todo = __ballot(le >= 0);
+  while (todo) {
+    const int v = __builtin_amdgcn_readlane(le, __builtin_ctzll(todo));
+    const uint64_t m = __ballot(le == v);
+    if (le == v) rank = __popcll(m & lt);
+    if (lane == 0) cnt[v] = __popcll(m);
+    todo &= ~m;
+  }
+  return rank;
+}
+
 // Routing of token t by one wavefront (kernel.py:428-542), for small batches: lane l holds
 // experts 4l..4l+3, so group g (32 experts) is lanes 8g..8g+7, and every lane does a quarter
 // of route_wave's per-token work. The selections are route_wave's: the same argmax keys, the

@@ -154,17 +154,8 @@ __device__ __forceinline__ int local_of(int id, int offset) {
 // (lower thread index first), plus per-expert counts. Up to 16 wavefronts, one slot per
 // thread (le < 0: not local). s_wcnt is [16][32] scratch; s_cnt receives the counts.
 __device__ __forceinline__ int block_rank(int le, int nwaves, int (*s_wcnt)[kExpertsLocal], int* s_cnt) {
-  const int lane = lane_id();
   const int wave = threadIdx.x >> 6;
-  const uint64_t lt = lanemask_lt();
-  int rank = 0, cnt = 0;
-#pragma unroll 4
-  for (int e = 0; e < kExpertsLocal; ++e) {
-    const uint64_t m = __ballot(le == e);
-    if (le == e) rank = __popcll(m & lt);
-    if (lane == e) cnt = __popcll(m);
-  }
-  if (lane < kExpertsLocal) s_wcnt[wave][lane] = cnt;
+  const int rank = wave_rank(le, s_wcnt[wave]);
   __syncthreads();
   if (threadIdx.x < kExpertsLocal) {
     int run = 0;
@@ -185,12 +176,7 @@ __device__ __forceinline__ int block_rank(int le, int nwaves, int (*s_wcnt)[kExp
 // (equal sizes rounded up to 16). Item = (expert, first row, rows,
 // first item of the expert | items of the expert << 16).
 __device__ __forceinline__ void finish_counts(const RouteParams& p, int e, int run, int* s_start) {
-  int incl = run;
-#pragma unroll
-  for (int off = 1; off < 32; off <<= 1) {
-    const int o = __shfl_up(incl, off, 32);
-    if (e >= off) incl += o;
-  }
+  const int incl = scan32(run);
   p.expert_count[e] = run;
   p.expert_start[e + 1] = incl;
   s_start[e + 1] = incl;
@@ -203,12 +189,7 @@ __device__ __forceinline__ void finish_counts(const RouteParams& p, int e, int r
     chunk = min(bm, (((run + nmax - 1) / nmax) + 15) & ~15);
   }
   const int nch = (run + chunk - 1) / chunk;
-  int ich = nch;
-#pragma unroll
-  for (int off = 1; off < 32; off <<= 1) {
-    const int o = __shfl_up(ich, off, 32);
-    if (e >= off) ich += o;
-  }
+  const int ich = scan32(nch);
   const int first = ich - nch;
   const int start = incl - run;
   for (int c = 0; c < nch; ++c) {
@@ -224,8 +205,9 @@ __device__ __forceinline__ void finish_counts(const RouteParams& p, int e, int r
   // rows (ties by expert index), experts without rows last. Their claim counters restart.
   const int key = nch > 0 ? min(chunk, run) : 0;
   int rank = 0;
+#pragma unroll
   for (int o = 0; o < kExpertsLocal; ++o) {
-    const int ko = __shfl(key, o, 32);
+    const int ko = __builtin_amdgcn_readlane(key, o);
     rank += (ko > key || (ko == key && o < e)) ? 1 : 0;
   }
   p.counters[kCtrOrder + rank] = first | (nch << 16);
@@ -297,6 +279,7 @@ static_assert(kWideParts == 4 && kWideTokens * kTopK <= 64, "one byte per part, 
 __global__ __launch_bounds__(kWideTokens * 64) void route_parts_kernel(RouteParams p) {
   __shared__ __attribute__((aligned(16))) float s_bias[kExpertsGlobal];
   __shared__ int s_le[kWideTokens * kTopK];
+  __shared__ int s_cnt[kExpertsLocal];
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int wave = tid >> 6;
@@ -324,18 +307,11 @@ __global__ __launch_bounds__(kWideTokens * 64) void route_parts_kernel(RoutePara
   __syncthreads();
   if (wave != 0) return;
   const int my_le = lane < kWideTokens * kTopK ? s_le[lane] : -1;
-  const uint64_t lt = lanemask_lt();
-  int rank = 0, cnt = 0;
-#pragma unroll 4
-  for (int e = 0; e < kExpertsLocal; ++e) {
-    const uint64_t me = __ballot(my_le == e);
-    if (my_le == e) rank = __popcll(me & lt);
-    if (lane == e) cnt = __popcll(me);
-  }
+  const int rank = wave_rank(my_le, s_cnt);
   if (my_le >= 0) p.slot_rank[blockIdx.x * kWideTokens * kTopK + lane] = rank;
   if (lane < kExpertsLocal)
     reinterpret_cast<uint8_t*>(p.block_count)[((blockIdx.x / kWideParts) * kExpertsLocal + lane) * 4 +
-                                              blockIdx.x % kWideParts] = (uint8_t)cnt;
+                                              blockIdx.x % kWideParts] = (uint8_t)s_cnt[lane];
 }
 
 // Routing of up to kSinglePassTokens tokens, one token per wavefront and four per work-group
@@ -471,13 +447,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(RouteParams p) {
     if (b == 0) {
       finish_counts(p, tid, te, s_start);
     } else {
-      int incl = te;
-#pragma unroll
-      for (int off = 1; off < kExpertsLocal; off <<= 1) {
-        const int o = __shfl_up(incl, off, kExpertsLocal);
-        if (tid >= off) incl += o;
-      }
-      s_start[tid + 1] = incl;
+      s_start[tid + 1] = scan32(te);
       if (tid == 0) s_start[0] = 0;
     }
   }
