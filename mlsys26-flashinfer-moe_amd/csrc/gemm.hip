@@ -555,7 +555,6 @@ __device__ __forceinline__ void fused_dispatch(const GemmParams& p, const RouteP
   const int wave = tid >> 6;
   const bool writer = blockIdx.x == 0;
   const int nslots = p.T * kTopK;
-  const uint64_t lt = lanemask_lt();
   int le[kFusedHalves], rank[kFusedHalves];
 #pragma unroll
   for (int h = 0; h < kFusedHalves; ++h) {
@@ -563,21 +562,10 @@ __device__ __forceinline__ void fused_dispatch(const GemmParams& p, const RouteP
     const int l = (slot < nslots ? ids[slot] : -1) - p.offset;
     le[h] = slot < nslots && l >= 0 && l < kExpertsLocal ? l : -1;
   }
-  // stable rank of each slot among the wavefront's slots of its expert, per-wavefront counts:
-  // one ballot per distinct local expert of the wavefront (a few at decode sizes)
+  // stable rank of each slot among the wavefront's slots of its expert, per-wavefront counts
 #pragma unroll
   for (int h = 0; h < kFusedHalves; ++h) {
-    int* cnt = s.cnt[h * kStreamWaves + wave];
-    if (lane < kExpertsLocal) cnt[lane] = 0;
-    rank[h] = 0;
-    uint64_t todo = __ballot(le[h] >= 0);
-    while (todo) {
-      const int v = __builtin_amdgcn_readlane(le[h], __builtin_ctzll(todo));
-      const uint64_t m = __ballot(le[h] == v);
-      if (le[h] == v) rank[h] = __popcll(m & lt);
-      if (lane == 0) cnt[v] = __popcll(m);
-      todo &= ~m;
-    }
+    rank[h] = wave_rank(le[h], s.cnt[h * kStreamWaves + wave]);
     if (writer) {
       // the 8 slots of a token are 8 consecutive lanes
       const uint64_t m = __ballot(le[h] >= 0);

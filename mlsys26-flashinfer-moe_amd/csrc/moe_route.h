@@ -85,23 +85,24 @@ __device__ __forceinline__ int scan32(int v) {
 
 // Stable rank of each lane's slot among the wavefront's slots of the same local expert (le < 0: not
 // local), and the wavefront's 32 counts in `cnt` (LDS): one ballot per distinct local expert of the
-// wavefront, a few of the 32 as a rule. Against a ballot for each of the 32 (with the scans by
-// shuffle): layer at T=80 162.0 -> 160.8 us, 128 168.7 -> 167.4, 901 239.4 -> 238.8, 8192 583.8 -> 582.2,
-// skewed T=128 220.0 -> 218.7. GEMM1's own dispatch keeps its shuffles: with scan32 T=16 68.7 -> 68.5,
-// but skewed T=64 170.4 -> 170.8.
+// wavefront, a few of the 32 as a rule. Lane e < 32 gathers expert e's count in a register and stores
+// cnt[e] itself, so that it may read it back at once; the other lanes' counts need a barrier. Against
+// a ballot for each of the 32 (with the scans by shuffle): layer at T=80 162.0 -> 160.8 us, 128
+// 168.7 -> 167.4, 901 239.4 -> 238.8, 8192 583.8 -> 582.2, skewed T=128 220.0 -> 218.7. GEMM1's own
+// dispatch keeps its scans by shuffle: with scan32 T=16 68.7 -> 68.5, but skewed T=64 170.4 -> 170.8.
 __device__ __forceinline__ int wave_rank(int le, int* cnt) {
   const int lane = lane_id();
   const uint64_t lt = lanemask_lt();
-  if (lane < kExpertsLocal) cnt[lane] = 0;
-  int rank = 0;
+  int rank = 0, n = 0;
   uint64_t todo = __ballot(le >= 0);
   while (todo) {
     const int v = __builtin_amdgcn_readlane(le, __builtin_ctzll(todo));
     const uint64_t m = __ballot(le == v);
     if (le == v) rank = __popcll(m & lt);
-    if (lane == 0) cnt[v] = __popcll(m);
+    if (lane == v) n = __popcll(m);
     todo &= ~m;
   }
+  if (lane < kExpertsLocal) cnt[lane] = n;
   return rank;
 }
 
