@@ -830,7 +830,8 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
   const int nsteps = n_items * kSliceSteps;
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
   // requant_kernel's operations on 4 columns per thread, 16 lanes per block. A wavefront's threads
-  // hold exactly the 256 columns of its own K-steps, so nothing is shared between wavefronts.
+  // hold exactly the 256 columns of its own K-steps, so nothing is shared between wavefronts; its
+  // lanes read each other's stores, hence the fence.
   static_assert(kSliceSteps * 128 == 64 * 4 && kQuantCols == 16 * 4, "columns of a wavefront");
   auto requantise = [&]() __attribute__((always_inline)) {
     const int tid = threadIdx.x;
@@ -868,6 +869,7 @@ __global__ __launch_bounds__(kSliceParts * 64) void gemm2_slice_kernel(GemmParam
         }
       }
     }
+    wave_lds_fence();
   };
   for (int slice = blockIdx.x; slice < kHiddenSlices; slice += gridDim.x) {
     const int h0 = slice * kSliceRows;

@@ -104,4 +104,13 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return l == 0 ? 0ull : (~0ull >> (64 - l));
 }
 
+// Orders a wavefront's LDS accesses across its lanes: what any lane stored before is what every lane loads
+// after. The hardware keeps a wavefront's LDS accesses in order, so this costs no wait; it keeps the
+// compiler from moving or forwarding them across.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace moe
