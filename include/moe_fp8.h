@@ -183,14 +183,16 @@ int moe_fp8_workspace_init(void* workspace, size_t workspace_bytes, hipStream_t 
 
 /* The whole layer: routing, dispatch, GEMM1+SwiGLU+requant, GEMM2+weighted combine.
  * Up to 64 tokens the dispatch is rebuilt inside the GEMM1 kernel instead of launched
- * before it; afterwards the workspace holds the same dispatch arrays as after the stage
- * entry points. Replaces run() (kernel.py:562-729). */
+ * before it, up to 4 tokens that kernel routes too, and with 1 token (2 on packed weights) the
+ * GEMM2 kernel requantises; afterwards the workspace holds the same dispatch arrays, act and
+ * act_scale as after the stage entry points. Replaces run() (kernel.py:562-729). */
 int moe_fp8_run(const moe_fp8_args* args, void* workspace, size_t workspace_bytes,
                 hipStream_t stream);
 
 /* moe_fp8_run with stage timing: the same launches, with events[0] recorded on `stream` before
  * stage 1 (routing, and the dispatch above 64 tokens), events[1] before stage 2 (GEMM1, one
- * kernel; up to 64 tokens it also rebuilds the dispatch), events[2] before stage 3
+ * kernel; up to 64 tokens it also rebuilds the dispatch, up to 4 it routes too and stage 1 is
+ * empty), events[2] before stage 3
  * (requantisation, GEMM2 and the combine) and events[3] after it. The events must have been
  * created by the caller (hipEventCreate) on the stream's device. With a non-NULL `packed` (the
  * packed copy of args' weights, moe_fp8_pack_weights) it times moe_fp8_run_packed instead.

@@ -202,7 +202,8 @@ namespace {
 
 // The launch sequence of moe_fp8_run; with `events`, events[i] is recorded on the stream
 // before stage i+1 (routing [+ dispatch], GEMM1, requantisation + GEMM2 + combine) and
-// events[3] after the last launch.
+// events[3] after the last launch, the launches being the same: a stage that another one's kernel
+// covers is empty.
 // packed: the packed copy of W13 and W2 (moe_fp8_pack_weights) or null; read only up to 256
 // tokens (MOE_FP8_PACKED_MAX_TOKENS), where the streaming kernels read it instead of args'
 // weights.
@@ -225,16 +226,15 @@ int run_layer(const moe_fp8_args* args, void* workspace, size_t workspace_bytes,
   if (!mark(0)) return MOE_FP8_ELAUNCH;
   if (args->num_tokens <= kFusedDispatchTokens) {
     // routing, then GEMM1 with the dispatch rebuilt in every work-group: one launch less
-    // (the smallest batches are routed there too, unless routing is timed as a stage)
-    const bool route = !events && gemm1_dispatch_routes(args->num_tokens);
-    if (!route && launch_route(rp, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
+    // (the smallest batches are routed there too)
+    if (!gemm1_dispatch_routes(args->num_tokens) && launch_route(rp, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
     if (!mark(1)) return MOE_FP8_ELAUNCH;
-    if (launch_gemm1_dispatch(gp, rp, use_packed, route, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
+    if (launch_gemm1_dispatch(gp, rp, use_packed, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
   } else {
     if (launch_route_dispatch(rp, stream) != hipSuccess || !mark(1)) return MOE_FP8_ELAUNCH;
     if (launch_gemm1(gp, L.rows_per_item, use_packed, stream) != hipSuccess || !mark(2)) return MOE_FP8_ELAUNCH;
   }
-  const bool requant = !events && gemm2_requantises(args->num_tokens, use_packed);
+  const bool requant = gemm2_requantises(args->num_tokens, use_packed);
   if (!requant && launch_requant(gp, L.rows_per_item, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
   if (launch_gemm2(gp, L.rows_per_item, use_packed, requant, stream) != hipSuccess) return MOE_FP8_ELAUNCH;
   if (launch_combine(gp, L.rows_per_item, stream) != hipSuccess || !mark(3)) return MOE_FP8_ELAUNCH;

@@ -1220,21 +1220,20 @@ bool gemm1_dispatch_routes(int T) { return T <= kInlineRouteTokens; }
 
 // Batches of up to kDeepRingTokens tokens: the ring's depth and whether the kernel routes.
 template <bool PACKED>
-hipError_t launch_gemm1_deep(const GemmParams& p, const RouteParams& rp, bool route, hipStream_t s) {
-  static std::atomic<int> occ[4] = {};
+hipError_t launch_gemm1_deep(const GemmParams& p, const RouteParams& rp, hipStream_t s) {
+  static std::atomic<int> occ[3] = {};
   static_assert(kDeeperRingTokens <= kInlineRouteTokens && kInlineRouteTokens <= kDeepRingTokens, "instances below");
   if (p.T <= kDeeperRingTokens)
-    return route ? launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeeperRing, true>, occ[0], p, rp, s)
-                 : launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeeperRing, false>, occ[1], p, rp, s);
-  return route ? launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, true>, occ[2], p, rp, s)
-               : launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, false>, occ[3], p, rp, s);
+    return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeeperRing, true>, occ[0], p, rp, s);
+  if (gemm1_dispatch_routes(p.T))
+    return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, true>, occ[1], p, rp, s);
+  return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, false>, occ[2], p, rp, s);
 }
 
-hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, bool packed, bool route, hipStream_t s) {
+hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, bool packed, hipStream_t s) {
   static std::atomic<int> occ_packed{0}, occ_rows{0};
   if (p.T <= 0 || p.T > kFusedDispatchTokens || rp.rows_per_item != kFusedItemRows) return hipErrorInvalidValue;
-  if (route && p.T > kInlineRouteTokens) return hipErrorInvalidValue;
-  if (p.T <= kDeepRingTokens) return packed ? launch_gemm1_deep<true>(p, rp, route, s) : launch_gemm1_deep<false>(p, rp, route, s);
+  if (p.T <= kDeepRingTokens) return packed ? launch_gemm1_deep<true>(p, rp, s) : launch_gemm1_deep<false>(p, rp, s);
   if (packed) return launch_dispatch_instance(gemm1_stream_dispatch_kernel<true>, occ_packed, p, rp, s);
   return launch_dispatch_instance(gemm1_stream_dispatch_kernel<false>, occ_rows, p, rp, s);
 }

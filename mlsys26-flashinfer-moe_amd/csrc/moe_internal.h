@@ -155,8 +155,8 @@ hipError_t launch_route(const RouteParams& p, hipStream_t s);
 // packed (items of up to 32 rows): p.w13 is the packed copy of W13 (moe_fp8_pack_weights).
 hipError_t launch_gemm1(const GemmParams& p, int rows_per_item, bool packed, hipStream_t s);
 // packed: p.w13 is the packed copy of W13 (moe_fp8_pack_weights).
-// route: the kernel routes the batch too (where gemm1_dispatch_routes(T)), without launch_route before it.
-hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, bool packed, bool route, hipStream_t s);
+// Where gemm1_dispatch_routes(T) the kernel routes the batch too, without launch_route before it.
+hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, bool packed, hipStream_t s);
 bool gemm1_dispatch_routes(int T);
 hipError_t launch_requant(const GemmParams& p, int rows_per_item, hipStream_t s);
 // packed (items of up to 32 rows): p.w2 is the packed copy of W2.

@@ -1,9 +1,9 @@
 """The smallest batches through moe_fp8_run and moe_fp8_run_packed, whose GEMM1 work-groups route the
 tokens themselves (up to 4) on rings of their own depth (6 slots up to 2 tokens, 4 up to 8), and whose
 GEMM2 work-groups requantise GEMM1's rows (1 token, packed 2): the top-k lists against the oracle,
-lists, dispatch and output bit for bit against moe_fp8_run_profiled, which routes in a launch of its
-own, and the requantised rows bit for bit against the formula and the output against the same
-tokens in a larger batch, which requant_kernel requantises."""
+lists, dispatch and output bit for bit against the stage entry points, which route, dispatch and
+requantise in launches of their own, and the requantised rows bit for bit against the formula and
+the output against the same tokens in a larger batch, which requant_kernel requantises."""
 import ctypes
 
 import numpy as np
@@ -25,20 +25,23 @@ def _weights():
     return gh, _STATE["w"], _STATE["p"]
 
 
-def _call(gh, args, ws, packed, profiled):
+def _call(gh, args, ws, packed, how="run"):
     lib = gh._lib.load()
     p, n = (packed.data_ptr(), packed.numel()) if packed is not None else (None, 0)
-    if profiled:
+    if how == "stages":
+        gh.route_dispatch(args, ws)
+        gh.gemm1(args, ws)
+        gh.gemm2_combine(args, ws)
+    elif how == "profiled":
         events = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
         for e in events:
             e.record()
-        rc = lib.moe_fp8_run_profiled(args, p, n, ws.ptr, ws.buffer.numel(), gh.stream(),
-                                      (ctypes.c_void_p * 4)(*[e.cuda_event for e in events]))
+        gh._lib.check(lib.moe_fp8_run_profiled(args, p, n, ws.ptr, ws.buffer.numel(), gh.stream(),
+                                               (ctypes.c_void_p * 4)(*[e.cuda_event for e in events])), how)
     elif packed is not None:
-        rc = lib.moe_fp8_run_packed(args, p, n, ws.ptr, ws.buffer.numel(), gh.stream())
+        gh._lib.check(lib.moe_fp8_run_packed(args, p, n, ws.ptr, ws.buffer.numel(), gh.stream()), how)
     else:
-        rc = lib.moe_fp8_run(args, ws.ptr, ws.buffer.numel(), gh.stream())
-    gh._lib.check(rc, "run")
+        gh.run_layer(args, ws)
 
 
 @pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16, torch.float16])
@@ -58,20 +61,19 @@ def test_small_batches(T, bias_dtype):
         if extreme:
             bias = bias.float().masked_fill(torch.arange(256, device=dev) >= 40, float("-inf")).to(bias_dtype)
         want = None
-        for pk in (None, packed):
-            for profiled in (True, False):
-                out = torch.full((T, 7168), 7.0, dtype=torch.bfloat16, device=dev)
-                ws = gh.new_workspace(T, dev)
-                args = gh.make_args(logits, bias, hq, hs, w[0], w[1], w[2], w[3], 32, 2.5, out)
-                for _ in range(2):
-                    _call(gh, args, ws, pk, profiled)
-                torch.cuda.synchronize()
-                ids = gh.read(ws, "topk_ids", torch.int32, T * 8).reshape(T, 8)
-                tw = gh.read(ws, "topk_weights", torch.float32, T * 8).reshape(T, 8)
-                gh.check_dispatch(ws, ids, tw, 32, T)
-                got = (ids.tobytes(), tw.tobytes(), out.view(torch.int16).cpu().numpy().tobytes())
-                want = want or got
-                assert got == want, (T, extreme, pk is not None, profiled)
+        for pk, how in ((None, "stages"), (None, "run"), (None, "profiled"), (packed, "run"), (packed, "profiled")):
+            out = torch.full((T, 7168), 7.0, dtype=torch.bfloat16, device=dev)
+            ws = gh.new_workspace(T, dev)
+            args = gh.make_args(logits, bias, hq, hs, w[0], w[1], w[2], w[3], 32, 2.5, out)
+            for _ in range(2):
+                _call(gh, args, ws, pk, how)
+            torch.cuda.synchronize()
+            ids = gh.read(ws, "topk_ids", torch.int32, T * 8).reshape(T, 8)
+            tw = gh.read(ws, "topk_weights", torch.float32, T * 8).reshape(T, 8)
+            gh.check_dispatch(ws, ids, tw, 32, T)
+            got = (ids.tobytes(), tw.tobytes(), out.view(torch.int16).cpu().numpy().tobytes())
+            want = want or got
+            assert got == want, (T, extreme, pk is not None, how)
         oid, ow = orouting.route(logits.cpu().numpy(), bias.float().cpu().numpy(), 2.5)
         assert np.array_equal(ids, oid) and np.array_equal(tw.view(np.uint32), ow.view(np.uint32))
 
@@ -92,7 +94,7 @@ def test_requantised_rows(T, boosted):
             args = gh.make_args(logits[:n].contiguous(), bias, hq[:n].contiguous(), hs[:, :n].contiguous(),
                                 w[0], w[1], w[2], w[3], 32, 2.5, out)
             for _ in range(2):
-                _call(gh, args, ws, pk, False)
+                _call(gh, args, ws, pk)
             torch.cuda.synchronize()
             outs.append(out)
             rows = int(gh.read(ws, "counters", torch.int32, 2)[1])
