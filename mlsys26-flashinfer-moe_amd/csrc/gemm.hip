@@ -645,9 +645,15 @@ __device__ __forceinline__ void fused_dispatch(const GemmParams& p, const RouteP
 // the bound of 8 tokens. 4 / 6 / 8 slots: 2 experts (256 units) 30.4 / 28.4 / 28.0 and 30.3 /
 // 27.9 / 27.9, 3 experts 36.3 / 35.9 / 36.5, 5 experts 49.9 / 50.8 / 51.7: 6 slots up to 2
 // tokens. The same depths on the row-major weights, 2 slots -> these: T=1 40.9 -> 35.8, T=2 44.5 ->
-// 40.8, T=3 47.8 -> 46.1, T=4 53.0 -> 50.9, T=5 55.0 -> 54.4, T=6 and T=8 within 0.4.
-// Bit-identical to the 2-slot ring.
+// 40.8, T=3 47.8 -> 46.1, T=4 53.0 -> 50.9; 6 / 4 slots at T=1 with 2, 3, 4, 6, 8 experts 30.5 / 33.1,
+// 36.9 / 38.6, 43.2 / 42.5, 57.2 / 56.2, 70.7 / 69.4 (one token seldom has more than 4); three tokens that
+// touch 19 experts lose, 153.4 -> 155.2. From 5
+// tokens they stay at 2 slots: four, which leave room for two work-groups per CU, gain with up to 4
+// experts and lose from 6 on, 2 -> 4 slots at T=5..8 with 2, 3, 4, 6, 7 experts 39.1 -> 35.7, 44.0 -> 41.0,
+// 48.0 -> 46.6, 57.6 -> 58.2, 64.2 -> 65.2 and T=5 with 22 experts 171 -> 175, and such batches are as
+// likely and every skewed one is among them. Bit-identical to the 2-slot ring.
 constexpr int kDeepRingTokens = 8;
+constexpr int kDeepRingRowTokens = 4;   // on row-major weights
 constexpr int kDeepRing = 4;
 constexpr int kDeeperRingTokens = 2;
 constexpr int kDeeperRing = 6;
@@ -678,7 +684,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void gemm1_stream_dispatch_kerne
   gemm1_stream_dispatch<PACKED, 0, false>(p, rp);
 }
 
-// The same on a RING-slot ring (batches of up to kDeepRingTokens tokens).
+// The same on a RING-slot ring (batches of up to kDeepRingTokens tokens, row-major kDeepRingRowTokens).
 template <bool PACKED, int RING, bool ROUTE>
 __global__ __launch_bounds__(kStreamWaves * 64) void gemm1_stream_dispatch_deep_kernel(GemmParams p, RouteParams rp) {
   gemm1_stream_dispatch<PACKED, RING, ROUTE>(p, rp);
@@ -1218,22 +1224,23 @@ hipError_t launch_dispatch_instance(K kernel, std::atomic<int>& occ, const GemmP
 
 bool gemm1_dispatch_routes(int T) { return T <= kInlineRouteTokens; }
 
-// Batches of up to kDeepRingTokens tokens: the ring's depth and whether the kernel routes.
+// Batches that the kernel routes too: the ring's depth.
 template <bool PACKED>
-hipError_t launch_gemm1_deep(const GemmParams& p, const RouteParams& rp, hipStream_t s) {
-  static std::atomic<int> occ[3] = {};
-  static_assert(kDeeperRingTokens <= kInlineRouteTokens && kInlineRouteTokens <= kDeepRingTokens, "instances below");
+hipError_t launch_gemm1_routed(const GemmParams& p, const RouteParams& rp, hipStream_t s) {
+  static std::atomic<int> occ[2] = {};
   if (p.T <= kDeeperRingTokens)
     return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeeperRing, true>, occ[0], p, rp, s);
-  if (gemm1_dispatch_routes(p.T))
-    return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, true>, occ[1], p, rp, s);
-  return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, false>, occ[2], p, rp, s);
+  return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<PACKED, kDeepRing, true>, occ[1], p, rp, s);
 }
 
 hipError_t launch_gemm1_dispatch(const GemmParams& p, const RouteParams& rp, bool packed, hipStream_t s) {
-  static std::atomic<int> occ_packed{0}, occ_rows{0};
+  static std::atomic<int> occ_deep{0}, occ_packed{0}, occ_rows{0};
+  static_assert(kDeeperRingTokens <= kInlineRouteTokens && kInlineRouteTokens <= kDeepRingTokens &&
+                kDeepRingRowTokens == kInlineRouteTokens, "instances below");
   if (p.T <= 0 || p.T > kFusedDispatchTokens || rp.rows_per_item != kFusedItemRows) return hipErrorInvalidValue;
-  if (p.T <= kDeepRingTokens) return packed ? launch_gemm1_deep<true>(p, rp, s) : launch_gemm1_deep<false>(p, rp, s);
+  if (gemm1_dispatch_routes(p.T)) return packed ? launch_gemm1_routed<true>(p, rp, s) : launch_gemm1_routed<false>(p, rp, s);
+  if (packed && p.T <= kDeepRingTokens)
+    return launch_dispatch_instance(gemm1_stream_dispatch_deep_kernel<true, kDeepRing, false>, occ_deep, p, rp, s);
   if (packed) return launch_dispatch_instance(gemm1_stream_dispatch_kernel<true>, occ_packed, p, rp, s);
   return launch_dispatch_instance(gemm1_stream_dispatch_kernel<false>, occ_rows, p, rp, s);
 }

@@ -1,5 +1,5 @@
 """The smallest batches through moe_fp8_run and moe_fp8_run_packed, whose GEMM1 work-groups route the
-tokens themselves (up to 4) on rings of their own depth (6 slots up to 2 tokens, 4 up to 8), and whose
+tokens themselves (up to 4) on rings of their own depth (6 slots up to 2 tokens, 4 up to 4, packed 8), and whose
 GEMM2 work-groups requantise GEMM1's rows (1 token, packed 2): the top-k lists against the oracle,
 lists, dispatch and output bit for bit against the stage entry points, which route, dispatch and
 requantise in launches of their own, and the requantised rows bit for bit against the formula and

@@ -43,3 +43,16 @@ def test_a_profiled_call_makes_the_launches_of_an_unprofiled_one(launches, T, pa
     assert marks == ["E0", "E1", "E2", "E3"] and timed[0] == "E0" and timed[-1] == "E3"
     gemm1 = timed[timed.index("E1") + 1:timed.index("E2")]
     assert len(gemm1) == 1 and gemm1[0].startswith(("gemm1_stream_dispatch", "gemm_stream_kernel<1", "gemm_tile_kernel<true"))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8, 9, 64])
+def test_the_ring_of_gemm1(launches, T, packed):
+    """6 slots up to 2 tokens, 4 up to 4 (packed 8), where 4 lose on the row-major weights with 6 experts or
+    more; the kernel routes up to 4 tokens."""
+    (rc, seq), = launches((T, packed, False, 0))
+    slots = 6 if T <= 2 else 4 if T <= (8 if packed else 4) else 0
+    p = str(packed).lower()
+    gemm1 = f"gemm1_stream_dispatch_deep_kernel<{p},{slots},{str(T <= 4).lower()}>" if slots else f"gemm1_stream_dispatch_kernel<{p}>"
+    assert rc == 0 and [x.split("@")[0] for x in seq if x.startswith("gemm1")] == [gemm1]
+    assert any(x.startswith("route") for x in seq) == (T > 4)
