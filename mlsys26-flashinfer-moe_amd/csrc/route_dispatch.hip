@@ -523,7 +523,8 @@ hipError_t launch_route(const RouteParams& p, hipStream_t s) { return launch_rou
 
 hipError_t launch_route_dispatch(const RouteParams& p, hipStream_t s) {
   if (p.single_pass) {
-    if (!p.skip_routing && launch_route_lists(p, s) != hipSuccess) return hipGetLastError();
+    const hipError_t rc = p.skip_routing ? hipSuccess : launch_route_lists(p, s);
+    if (rc != hipSuccess) return rc;
     hipLaunchKernelGGL(dispatch_small_kernel, dim3(1), dim3(kRouteThreads), 0, s, p);
   } else if (p.T <= kWideDispatchTokens) {
     hipLaunchKernelGGL(route_parts_kernel, dim3(p.nblocks * kWideParts), dim3(kWideTokens * 64), 0, s, p);

@@ -56,3 +56,11 @@ def test_the_ring_of_gemm1(launches, T, packed):
     gemm1 = f"gemm1_stream_dispatch_deep_kernel<{p},{slots},{str(T <= 4).lower()}>" if slots else f"gemm1_stream_dispatch_kernel<{p}>"
     assert rc == 0 and [x.split("@")[0] for x in seq if x.startswith("gemm1")] == [gemm1]
     assert any(x.startswith("route") for x in seq) == (T > 4)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("T", SIZES)
+def test_a_failed_launch_is_reported(launches, T, packed):
+    (_, seq), = launches((T, packed, False, 0))
+    failed = launches(*[(T, packed, False, n) for n in range(1, len(seq) + 1)])
+    assert [rc for rc, _ in failed] == [-6] * len(seq)   # MOE_FP8_ELAUNCH
