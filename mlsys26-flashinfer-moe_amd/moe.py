@@ -331,15 +331,17 @@ def _run_direct(routing_logits, routing_bias, hidden_states, hidden_states_scale
     Returns False, having done nothing, for every other call: _run handles those (and raises
     what there is to raise). With _run's general path a decode call of one token was bound by its
     ~33 us of host time, the GPU's work taking 23."""
-    T = routing_logits.shape[0] if routing_logits.dim() == 2 else 0
-    bias_code = _BIAS_CODES.get(routing_bias.dtype)
     f32, fp8 = torch.float32, torch.float8_e4m3fn
-    if T == 0 or bias_code is None or not (
-            hidden_states.dtype is fp8 and gemm1_weights.dtype is fp8 and gemm2_weights.dtype is fp8
-            and routing_logits.dtype is f32 and hidden_states_scale.dtype is f32
+    # (in validate's order, so that what is no tensor meets the same assertion)
+    if not (hidden_states.dtype is fp8 and gemm1_weights.dtype is fp8 and gemm2_weights.dtype is fp8
+            and routing_logits.dtype is f32 and routing_bias.dtype in _BIAS_CODES and hidden_states_scale.dtype is f32
             and gemm1_weights_scale.dtype is f32 and gemm2_weights_scale.dtype is f32
             and (output.dtype is torch.bfloat16 or output.dtype is f32)):
         return False
+    T = routing_logits.shape[0] if routing_logits.dim() == 2 else 0
+    if T == 0:
+        return False
+    bias_code = _BIAS_CODES[routing_bias.dtype]
     # (the contract puts no shape on the bias; what is not [256] takes the general path)
     if not (routing_logits.shape[1] == EXPERTS_GLOBAL and routing_bias.shape == (EXPERTS_GLOBAL,)
             and hidden_states.shape == (T, HIDDEN) and hidden_states_scale.shape == (H_BLOCKS, T)

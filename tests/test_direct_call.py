@@ -1,5 +1,6 @@
 """run()'s and quantize_hidden()'s direct call (nothing moved, copied or converted) against their
 general path: which calls take it, and that both give the same bits."""
+import numpy as np
 import pytest
 import torch
 
@@ -39,6 +40,17 @@ def test_tensors_off_the_gpu_take_the_general_path(moe):
     assert not moe._run_direct(**_cpu_args(moe))
     assert not moe._run_direct(**_cpu_args(moe, T=0))
     assert not moe._quantize_direct(torch.zeros(2, 7168), torch.zeros(2, 7168).to(torch.float8_e4m3fn), torch.zeros(56, 2))
+
+
+@pytest.mark.parametrize("name, message", [
+    ("routing_logits", "routing_logits must be float32"), ("routing_bias", "routing_bias must be"),
+    ("hidden_states", "hidden_states must be"), ("hidden_states_scale", "hidden_states_scale must be"),
+    ("gemm1_weights", "gemm1_weights must be"), ("gemm2_weights_scale", "gemm2_weights_scale must be")])
+def test_an_array_in_place_of_a_tensor_meets_the_contracts_assertion(moe, name, message):
+    a = _cpu_args(moe, **{name: np.zeros((3, 256), dtype=np.float32)})
+    del a["packed"]
+    with pytest.raises(AssertionError, match=message):
+        moe.run(**a)
 
 
 def _off(t, elements):
