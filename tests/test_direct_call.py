@@ -118,4 +118,5 @@ def test_direct_quantiser_gives_the_general_paths_bits(moe, T, dtype):
         moe.quantize_hidden(src, out=q, out_scale=s)
         assert torch.equal(q.view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(s, want[1])
     assert not moe._quantize_direct(x, None, None)
+    assert not moe._quantize_direct(_off(x, 1), object(), object())   # declined before the outputs are looked at
     assert not moe._quantize_direct(x, _off(q.view(torch.uint8), 1).view(torch.float8_e4m3fn), s)
