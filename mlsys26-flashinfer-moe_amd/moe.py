@@ -18,6 +18,12 @@ from ._lib import (BIAS_BF16, BIAS_F16, BIAS_F32, EXPERTS_GLOBAL, EXPERTS_LOCAL,
                    H_BLOCKS, HIDDEN, HIDDEN_BF16, HIDDEN_F16, HIDDEN_F32, I_BLOCKS, INTER, OUT_BF16,
                    OUT_F32, PACKED_MAX_TOKENS)
 
+# The current device and a device's current stream handle without a device or stream object (a call of
+# one token is bound by its host time); torch's public functions where these are missing.
+_device_index = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+    (lambda device: torch.cuda.current_stream(device).cuda_stream)
+
 _BIAS_CODES = {torch.float32: BIAS_F32, torch.bfloat16: BIAS_BF16, torch.float16: BIAS_F16}
 
 
@@ -264,9 +270,8 @@ class PackedWeightCache:
 
 
 def _current_stream_id() -> int:
-    """The current stream's handle on the current device (torch.cuda.current_stream().cuda_stream
-    without the stream object)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    """The current stream's handle on the current device."""
+    return _raw_stream(_device_index())
 
 
 def _record_event():
@@ -351,7 +356,7 @@ def _run_direct(routing_logits, routing_bias, hidden_states, hidden_states_scale
             and gemm2_weights_scale.shape == (EXPERTS_LOCAL, H_BLOCKS, I_BLOCKS) and output.shape == (T, HIDDEN)):
         return False
     dev = output.get_device() if output.is_cuda else -1
-    if dev < 0 or torch._C._cuda_getDevice() != dev:
+    if dev < 0 or _device_index() != dev:
         return False
     ptrs = []
     for t in (routing_logits, routing_bias, hidden_states, hidden_states_scale, gemm1_weights, gemm1_weights_scale,
@@ -371,7 +376,7 @@ def _run_direct(routing_logits, routing_bias, hidden_states, hidden_states_scale
     if packed is not None and packed is not _AUTO and packed.device != output.device:
         return False
     capturing = torch.cuda.is_current_stream_capturing()
-    stream = torch._C._cuda_getCurrentRawStream(dev)
+    stream = _raw_stream(dev)
     ws = _workspaces.get((dev, stream), T, _layer_bytes(T), output.device, None, capturing)
     if packed is _AUTO:
         packed = _packed_weights.get(gemm1_weights, gemm2_weights, capturing) if T <= PACKED_MAX_TOKENS else None
@@ -519,7 +524,7 @@ def _quantize_direct(x, out, out_scale) -> bool:
     if out is None or out_scale is None or code is None or not x.is_cuda or x.data_ptr() & 15 or x.dim() != 2:
         return False
     T, dev = x.shape[0], x.get_device()
-    if not (T > 0 and x.shape[1] == HIDDEN and x.is_contiguous() and torch._C._cuda_getDevice() == dev
+    if not (T > 0 and x.shape[1] == HIDDEN and x.is_contiguous() and _device_index() == dev
             and out.dtype is torch.float8_e4m3fn and out.shape == (T, HIDDEN) and out.is_cuda
             and out.get_device() == dev and out.is_contiguous()
             and out_scale.dtype is torch.float32 and out_scale.shape == (H_BLOCKS, T) and out_scale.is_cuda
@@ -528,7 +533,7 @@ def _quantize_direct(x, out, out_scale) -> bool:
     px, pq, ps = x.data_ptr(), out.data_ptr(), out_scale.data_ptr()
     if pq & 7 or ps & 3:
         return False
-    _lib.check(_lib.load().moe_fp8_quantize_hidden(px, code, T, pq, ps, torch._C._cuda_getCurrentRawStream(dev)),
+    _lib.check(_lib.load().moe_fp8_quantize_hidden(px, code, T, pq, ps, _raw_stream(dev)),
                "moe_fp8_quantize_hidden")
     return True
 

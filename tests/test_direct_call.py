@@ -1,5 +1,8 @@
 """run()'s and quantize_hidden()'s direct call (nothing moved, copied or converted) against their
 general path: which calls take it, and that both give the same bits."""
+import importlib.util
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -34,6 +37,18 @@ def test_struct_bytes_are_the_ctypes_struct(moe):
     for (name, _), v in zip(_lib.MoeFp8Args._fields_, values):
         setattr(a, name, v)
     assert bytes(a) == moe._ARGS.pack(*values)
+
+
+def test_the_current_stream_without_torchs_private_functions(moe, monkeypatch):
+    for name in ("_cuda_getDevice", "_cuda_getCurrentRawStream"):
+        monkeypatch.delattr(torch._C, name, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: types.SimpleNamespace(cuda_stream=70 + device))
+    spec = importlib.util.spec_from_file_location(moe.__name__ + "_again", moe.__file__)
+    again = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(again)
+    assert again._current_stream_id() == 73
+    assert not again._run_direct(**_cpu_args(again))
 
 
 def test_tensors_off_the_gpu_take_the_general_path(moe):
