@@ -521,7 +521,10 @@ def _quantize_direct(x, out, out_scale) -> bool:
     contract's type and shape. Returns False, having done nothing, for every other call."""
     # (what the general path has to make or copy declines at once: 16.9 us there, 18.5 with every check before it)
     code = _HIDDEN_CODES.get(x.dtype)
-    if out is None or out_scale is None or code is None or not x.is_cuda or x.data_ptr() & 15 or x.dim() != 2:
+    if out is None or out_scale is None or code is None or not x.is_cuda or x.dim() != 2:
+        return False
+    px = x.data_ptr()
+    if px & 15:
         return False
     T, dev = x.shape[0], x.get_device()
     if not (T > 0 and x.shape[1] == HIDDEN and x.is_contiguous() and _device_index() == dev
@@ -530,7 +533,7 @@ def _quantize_direct(x, out, out_scale) -> bool:
             and out_scale.dtype is torch.float32 and out_scale.shape == (H_BLOCKS, T) and out_scale.is_cuda
             and out_scale.get_device() == dev and out_scale.is_contiguous()):
         return False
-    px, pq, ps = x.data_ptr(), out.data_ptr(), out_scale.data_ptr()
+    pq, ps = out.data_ptr(), out_scale.data_ptr()
     if pq & 7 or ps & 3:
         return False
     _lib.check(_lib.load().moe_fp8_quantize_hidden(px, code, T, pq, ps, _raw_stream(dev)),
