@@ -114,6 +114,7 @@ typedef struct moe_fp8_args {
  *   sorted_slot   int32 [N_max]     flat slot t*8+k of each assignment
  *   token_nlocal  int32 [T]         number of local assignments of each token
  *   slot_rank     int32 [T*8]       internal: the multi-work-group dispatch's stable ranks
+ *   block_count   int32 [route_blocks, 32]  internal: its expert histograms, of 16 tokens each
  *   work_items    int32 [max_items, 4]  GEMM work list (expert, first row, rows,
  *                                   first item of the expert | its item count << 16) (kernel.py:384-407)
  *   counters      int32 [96]        [0] number of work items, [1] N; the rest internal
@@ -133,8 +134,8 @@ typedef struct moe_fp8_args {
  *                                                                                     (kernel.py:704)
  *   swiglu        fp32  [N_max, 2048]    SwiGLU output before requantisation; only for
  *                                        T <= 256 (0 bytes otherwise)
- *   row_dest      int32 [N_max]     above 256 tokens, written by the dispatch: GEMM2's output
- *                                   destination of each bucket row, the token when it has one
+ *   row_dest      int32 [N_max]     above 128 tokens, written by the dispatch (and read above 256):
+ *                                   GEMM2's output destination of each bucket row, the token when it has one
  *                                   local assignment (its output row is written directly),
  *                                   else -1 - its flat slot (the row is parked in `partial`)
  */
@@ -160,7 +161,7 @@ typedef struct moe_fp8_layout {
   int32_t num_tokens;
   int32_t max_assignments;   /* N_max = 8*T        */
   int32_t max_work_items;
-  int32_t route_blocks;      /* routing work-groups */
+  int32_t route_blocks;      /* 16-token blocks of the routing */
   int32_t rows_per_item;     /* GEMM rows (assignments) per work item */
   int32_t requant_block;     /* columns per act_scale entry: 64 below 4096 tokens, else 128 */
   int32_t reserved[2];

@@ -779,12 +779,14 @@ constexpr int kSliceLdsDma = kSliceLdsRows / 8;                 // 4 DMA instruc
 // stream could not start; it costs every CU the fp32 rows' bytes and ~0.25 us per row. Layer,
 // us, few local rows (random routing) and many (every token names 5 to 8 local experts):
 //                 packed, random   many         row-major, random   many
-//   T=1           21.2 -> 19.5     43.4 -> 42.4     35.7 -> 34.8   46.4 -> 46.4
+//   T=1           21.2 -> 19.5     43.4 -> 42.4     35.7 -> 34.8   46.4 -> 46.4 (6 rows 57.1 -> 57.3, 8: 70.7 -> 71.7)
 //   T=2           36.9 -> 35.6     53.2 -> 53.2     40.5 -> 40.1   55.7 -> 57.5
 //   T=3           43.8 -> 42.9     55.6 -> 56.8     46.1 -> 46.1
 //   T=4           48.5 -> 47.7     58.5 -> 60.9     50.6 -> 50.9   59.1 -> 64.0
-// so up to the sizes at which many rows lose nothing: 2 tokens packed, 1 row-major (whose LDS
-// ring the compiler drains around the rows' LDS stores).
+// so up to the sizes at which many rows lose nothing, or next to nothing with the 6 or 8 rows that one
+// token seldom has here: 2 tokens packed, 1 row-major. On row-major weights the compiler drains the LDS
+// ring (vmcnt(0)) around the rows' stores, and again in every K-step, before it reads the act scales:
+// they share an LDS object with the ring's DMAs.
 constexpr int kSlicePackedTokens = 2;
 constexpr int kSliceRowMajorTokens = 1;
 constexpr int kSliceActStride = kInter + 16;   // the 16 rows of a fragment load fall in distinct banks

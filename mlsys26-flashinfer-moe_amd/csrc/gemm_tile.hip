@@ -334,8 +334,9 @@ __device__ __forceinline__ void tile_body(const GemmParams& p, const TileCtx<ROW
 
   // A step's loads are issued in up to this many pieces, spread over its row groups: eight wavefronts
   // that issue their seven loads at once right after the barrier wait for the address unit, all
-  // together, before their first MFMA (T=4000 layer 413 -> 402 us, skewed T=4096 batch 1152 -> 1125,
-  // T=8192 608 -> 598, T=14107 940 -> 921; with weights hot in the L2s a K-step took as long
+  // together, before their first MFMA (layer, whole loads -> pieces: 901 tokens 243 / 243 us, 2048
+  // 338.4 -> 333.4, 4000 435.5 -> 423.9, skewed 4096 1119 -> 1099, 8192 tokens with 7641 local rows 550.9 ->
+  // 541.0, 14107 with 18086 1131 -> 1109; with weights hot in the L2s a K-step took as long
   // as its loads alone and its MFMAs alone together). More pieces need more registers than the
   // 160-row instances have (GEMM1 in three spills 4, GEMM2 in two 11: no faster).
   constexpr int kMaxPieces = ROWS == kTileItemRowsMid ? 3 : G1 ? 2 : 1;
@@ -738,8 +739,10 @@ struct XcdList {
   // 1.8 MB 44-48 us), and a half takes half as long. In a fuller round the CUs share the HBM's
   // rate and halves only double the activation loads. Whole layer, whole / split: T=300 with 21
   // items (10 units over) 211 / 201 us, T=512 with 20 (8 over) 205 / 195, T=901 with 22 (12 over)
-  // 222 / 215, T=2048 with 33 (2 over) 329 / 318, T=512 with 24 (16 over, the most that are split)
-  // 221 / 216. Bit-identical.
+  // 222 / 215, T=2048 with 33 (2 over) 329 / 318. At 16 over, the most that are split, 84 random batches
+  // of 300 to 4095 tokens changed by -4.3..+3.1%, -0.9% on average (T=300 219.5 / 212.3, 4000 462 / 468; the
+  // worst 2048 tokens with few local rows, 239.8 / 247.3); without a split the two instances cost up
+  // to 0.5% (T=512 with 27 items 240.8 / 241.7). Bit-identical.
   __device__ __forceinline__ void split_tail(int work_groups) {
     const int r = total % work_groups;
     if (2 * r <= work_groups) {

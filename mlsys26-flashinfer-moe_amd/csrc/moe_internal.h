@@ -112,11 +112,15 @@ struct RouteParams {
   float* sorted_weight;
   int32_t* sorted_slot;
   int32_t* token_nlocal;
+  // [T*8] stable rank of each local slot: among its 16-token block's slots of the expert, or
+  // (route_parts_kernel) its 4-token quarter's
   int32_t* slot_rank;
   // [N_max] output destination of each bucket row for the tile GEMM2 (place_kernel): the token
   // when it has one local assignment, else -1 - its flat slot
   int32_t* row_dest;
-  int32_t* block_count;  // [nblocks, 32] expert histogram of each routing work-group
+  // [nblocks, 32] expert histogram of each 16-token block: its count, or (route_parts_kernel) the
+  // counts of its four quarters, one byte each
+  int32_t* block_count;
   int32_t* work_items;   // [max_items, 4]
   int32_t* counters;
 };

@@ -270,8 +270,9 @@ __global__ __launch_bounds__(kRouteWaves * 64) void route_kernel(RouteParams p) 
 // last token, so that every byte is written. What bounds it is the dependent chain of a token's
 // eight argmax rounds, on a chip that is mostly idle: four tokens per wavefront and 16 per
 // work-group make that chain longer and fill 57 CUs at 901 tokens, these 226. Layer, us,
-// against route_kernel: T=300 204.3 -> 202.1, 901 242.0 -> 240.2, 1500 268.0 -> 266.3, 2048 301.2 ->
-// 299.4; 3000 351.3 -> 352.0, 4000 397.6 -> 399.1 (2.5 times the instructions per token).
+// against route_kernel: T=129 182.2 -> 180.4, 256 194.8 -> 192.7, 300 202.8 -> 201.0, 901 243.9 -> 242.5, 1500
+// 277.8 -> 276.7, 2048 no difference (334.1 / 333.1, 311.6 / 311.7); 3000 329.1 -> 329.5, 4000 318.5 -> 319.4, 8192
+// 541.3 -> 544.1 (2.5 times the instructions per token).
 constexpr int kWideTokens = 4;
 constexpr int kWideParts = kRouteTokensPerBlock / kWideTokens;   // 4 bytes of an entry
 static_assert(kWideParts == 4 && kWideTokens * kTopK <= 64, "one byte per part, one wavefront's slots");
